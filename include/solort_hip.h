@@ -359,6 +359,28 @@ int solort_prefill_layer(const void* qkv, int64_t qkv_row_stride, int T, int nh,
 int solort_accept_prefix(const int64_t* target, const int64_t* draft, int k, int64_t* out, solort_stream_t stream);
 
 /*
+ * Residual sum and RMSNorm of m rows (prefill and verify; the token-by-token
+ * step has them inside solort_gemv): with y non-NULL x_out = x + y in bf16
+ * (cuda_graph_executor.py:131, :134, :264, :267; x_out may be x), then h =
+ * _rmsnorm(x_out, norm_w, eps) (:25-28) of that rounded sum; with y NULL h =
+ * _rmsnorm(x, norm_w, eps) and x_out is not used.  k a multiple of 8 up to
+ * 65536, row strides multiples of 8, everything 16-byte aligned; h must not
+ * overlap x, y or x_out.
+ */
+int solort_add_rmsnorm(const void* x, int64_t x_row_stride, const void* y, int64_t y_row_stride, const void* norm_w,
+                       float eps, int m, int k, void* x_out, int64_t x_out_row_stride, void* h, int64_t h_row_stride,
+                       solort_stream_t stream);
+
+/*
+ * out[r][i] = silu(gu[r][i]) * gu[r][inter + i] over m gate_up rows
+ * (cuda_graph_executor.py:132-134, :265-267), silu and the product each
+ * rounded to bf16.  inter and the row strides multiples of 8, 16-byte
+ * aligned, m <= 65535; out must not overlap gu.
+ */
+int solort_swiglu_rows(const void* gu, int64_t gu_row_stride, int m, int inter, void* out, int64_t out_row_stride,
+                       solort_stream_t stream);
+
+/*
  * Decode-step matrix-vector product around the attention block, one token:
  * W [rows][w_row_stride] bf16 row-major (torch Linear weight), x [k] bf16,
  * fp32 accumulation, bf16 out [n_out].  Replaces the T = 1 GEMMs of

@@ -75,13 +75,6 @@ class RandomQwen3:
         self.lm_head = self.embed if s.tie_embeddings else rnd(s.vocab, H)
 
 
-def _rmsnorm_rows(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
-    """cuda_graph_executor.py:25-28 over the rows of a prompt, as the reference's torch ops on the
-    device: fp32 upcast, x * rsqrt(mean(x^2) + eps), times w in fp32, cast back."""
-    xf = x.float()
-    return ((xf * torch.rsqrt(xf.square().mean(-1, keepdim=True) + eps)) * w.float()).to(x.dtype)
-
-
 class GraphQwen3Decode:
     """Greedy decode over a runner-owned bf16 KV cache, one captured graph per KV bucket."""
 
@@ -216,9 +209,11 @@ class GraphQwen3Decode:
         cs = self.cs_pre[: 2 * bound * (HD // 2)].view(2, bound, HD // 2)
         ops.rope_rows(self.inv_freq, self.zero_pos, bound, cs)                  # :111
         x = w.embed.index_select(0, self.pre_tok[:bound])                       # :112
+        h = torch.empty_like(x)
         ctx = self.ctx_pre[:bound]
+        ops.add_rmsnorm(x, None, w.in_ln[0], self.eps, None, h)                  # :114
         for li in range(s.layers):
-            qkv = F.linear(_rmsnorm_rows(x, w.in_ln[li], self.eps), w.wqkv[li])  # :114-115
+            qkv = F.linear(h, w.wqkv[li])                                        # :115
             if bound >= FUSED_PREFILL_MIN:                                       # :116-130
                 ops.prefill_layer(qkv, w.qn[li], w.kn[li], self.eps, cs, self.kc[li], self.vc[li], self.scale, ctx,
                                   s.nh, s.nkv)
@@ -226,10 +221,22 @@ class GraphQwen3Decode:
                 ops.qknorm_rope_kvwrite_cs(qkv, w.qn[li], w.kn[li], self.eps, cs, None, self.q_pre[:bound],
                                            self.kc[li], self.vc[li], s.nh, s.nkv)
                 ops.prefill_attn(self.q_pre[:bound], self.kc[li], self.vc[li], self.scale, ctx)
-            x = x + F.linear(ctx, w.wo[li])                                      # :131
-            gate, up = F.linear(_rmsnorm_rows(x, w.post_ln[li], self.eps), w.wgu[li]).split(s.inter, dim=-1)
-            x = x + F.linear(F.silu(gate) * up, w.wd[li])                        # :132-134
+            self._mlp_rows(li, x, h, ctx)                                        # :131-134
         return x
+
+    def _mlp_rows(self, li: int, x: torch.Tensor, h: torch.Tensor, ctx: torch.Tensor) -> None:
+        """The rest of layer li for the rows of ctx (cuda_graph_executor.py:131-134, :264-267): x gains the
+        layer's two residual terms, and h becomes the next layer's normalised input."""
+        s, w = self.s, self.w
+        ops.add_rmsnorm(x, F.linear(ctx, w.wo[li]), w.post_ln[li], self.eps, x, h)
+        gu = F.linear(h, w.wgu[li])
+        act = torch.empty(x.shape[0], s.inter, dtype=torch.bfloat16, device=self.dev)
+        ops.swiglu_rows(gu, act)
+        y = F.linear(act, w.wd[li])
+        if li + 1 < s.layers:
+            ops.add_rmsnorm(x, y, w.in_ln[li + 1], self.eps, x, h)
+        else:
+            x.add_(y)
 
     def prefill(self, ids: torch.Tensor | list[int]) -> None:
         """Graphed bucketed prefill (cuda_graph_executor.py:149-161) of a prompt of plen tokens: pads
@@ -286,14 +293,15 @@ class GraphQwen3Decode:
         s, w = self.s, self.w
         ops.rope_rows(self.inv_freq, self.vpos0, self.k1, self.cs_ver)          # :248
         x = w.embed.index_select(0, self.vtok)                                  # :249
+        h = torch.empty_like(x)
+        ops.add_rmsnorm(x, None, w.in_ln[0], self.eps, None, h)                  # :252
         for li in range(s.layers):
-            qkv = F.linear(_rmsnorm_rows(x, w.in_ln[li], self.eps), w.wqkv[li])  # :252-253
+            qkv = F.linear(h, w.wqkv[li])                                        # :253
             ops.decode_layer(qkv, w.qn[li], w.kn[li], self.eps, self.cs_ver, self.vpos0, self.kc[li], self.vc[li],
                              bound, self.scale, self.ws_ver, verify_splits(bound, s.nkv), self.ctx_ver, s.nh, s.nkv)
-            x = x + F.linear(self.ctx_ver, w.wo[li])                            # :264
-            gate, up = F.linear(_rmsnorm_rows(x, w.post_ln[li], self.eps), w.wgu[li]).split(s.inter, dim=-1)
-            x = x + F.linear(F.silu(gate) * up, w.wd[li])                       # :265-267
-        logits = F.linear(_rmsnorm_rows(x, w.final_norm, self.eps), w.lm_head)   # :268
+            self._mlp_rows(li, x, h, self.ctx_ver)                               # :264-267
+        ops.add_rmsnorm(x, None, w.final_norm, self.eps, None, h)
+        logits = F.linear(h, w.lm_head)                                          # :268
         ops.argmax_rows(logits, self.tok_ver, self.ws_argv)
         if self.k1 > 1:
             ops.accept_prefix(self.tok_ver, self.vtok[1:], self.acc_ver)

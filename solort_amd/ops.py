@@ -534,6 +534,43 @@ def accept_prefix(target: torch.Tensor, draft: torch.Tensor, out: torch.Tensor) 
     _lib.check(rc, "accept_prefix")
 
 
+def _rows(name: str, t: torch.Tensor, m: int, k: int) -> None:
+    _on_gpu(name, t, torch.bfloat16)
+    _need(t.shape == (m, k) and t.stride(1) == 1, f"{name} must be [{m}, {k}] with unit column stride")
+
+
+def add_rmsnorm(x: torch.Tensor, y: torch.Tensor | None, norm_w: torch.Tensor, eps: float,
+                x_out: torch.Tensor | None, h: torch.Tensor) -> None:
+    """x_out = x + y (x_out may be x), h = rmsnorm(x_out, norm_w) over the rows of x [m, k] bf16; with y
+    None h = rmsnorm(x, norm_w).  See solort_add_rmsnorm."""
+    _need(x.dim() == 2, "x must be [m, k]")
+    m, k = x.shape
+    _rows("x", x, m, k)
+    _rows("h", h, m, k)
+    _on_gpu("norm_w", norm_w, torch.bfloat16)
+    _need(norm_w.numel() == k and norm_w.is_contiguous(), f"norm_w must hold k = {k} values")
+    if y is not None:
+        _need(x_out is not None, "y needs x_out")
+        _rows("y", y, m, k)
+        _rows("x_out", x_out, m, k)
+    rc = _lib.load().solort_add_rmsnorm(
+        x.data_ptr(), x.stride(0), None if y is None else y.data_ptr(), 0 if y is None else y.stride(0),
+        norm_w.data_ptr(), float(eps), m, k, None if y is None else x_out.data_ptr(),
+        0 if y is None else x_out.stride(0), h.data_ptr(), h.stride(0), _stream(x))
+    _lib.check(rc, "add_rmsnorm")
+
+
+def swiglu_rows(gu: torch.Tensor, out: torch.Tensor) -> None:
+    """out [m, inter] = silu(gu[:, :inter]) * gu[:, inter:], bf16; see solort_swiglu_rows."""
+    _need(out.dim() == 2, "out must be [m, inter]")
+    m, inter = out.shape
+    _rows("out", out, m, inter)
+    _rows("gu", gu, m, 2 * inter)
+    rc = _lib.load().solort_swiglu_rows(gu.data_ptr(), gu.stride(0), m, inter, out.data_ptr(), out.stride(0),
+                                        _stream(gu))
+    _lib.check(rc, "swiglu_rows")
+
+
 GEMV_PLAIN, GEMV_RESID, GEMV_SWIGLU = 0, 1, 2
 
 
