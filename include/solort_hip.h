@@ -396,6 +396,18 @@ int solort_swiglu_rows(const void* gu, int64_t gu_row_stride, int m, int inter, 
 int solort_gemv(const void* w, int64_t w_row_stride, int n_out, int k, const void* x, const void* norm_w, float eps,
                 const void* res, int mode, int64_t inter, void* out, solort_stream_t stream);
 
+/*
+ * solort_gemv for m <= 16 rows (the K+1 tokens of a verify step, a short
+ * prompt): out[t] = W x[t], t < m, with the same fused neighbours and modes
+ * (norm_w: the RMSNorm of every x row; SOLORT_GEMV_RESID: res row t added, out
+ * may be res; SOLORT_GEMV_SWIGLU).  Replaces the T-row products of
+ * cuda_graph_executor.py:104-135 and :245-268.  Row strides in elements, of w
+ * and x multiples of 8; x must not overlap out.
+ */
+int solort_gemm_rows(const void* w, int64_t w_row_stride, int n_out, int k, const void* x, int64_t x_row_stride, int m,
+                     const void* norm_w, float eps, const void* res, int64_t res_row_stride, int mode, int64_t inter,
+                     void* out, int64_t out_row_stride, solort_stream_t stream);
+
 /* Workspace bytes for solort_gemv_argmax with n_out outputs (one 8-byte key
  * per workgroup; no zero-fill needed). */
 size_t solort_gemv_argmax_workspace_bytes(int n_out);

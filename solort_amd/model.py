@@ -225,7 +225,7 @@ class GraphQwen3Decode:
         return x
 
     def _mlp_rows(self, li: int, x: torch.Tensor, h: torch.Tensor, ctx: torch.Tensor) -> None:
-        """The rest of layer li for the rows of ctx (cuda_graph_executor.py:131-134, :264-267): x gains the
+        """The rest of layer li for the rows of ctx (cuda_graph_executor.py:131-134): x gains the
         layer's two residual terms, and h becomes the next layer's normalised input."""
         s, w = self.s, self.w
         ops.add_rmsnorm(x, F.linear(ctx, w.wo[li]), w.post_ln[li], self.eps, x, h)
@@ -286,22 +286,24 @@ class GraphQwen3Decode:
         return self._read_tokens(n)
 
     def _verify_forward(self, bound: int) -> torch.Tensor:
-        """cuda_graph_executor.py:245-268 for the k1 tokens in vtok at vpos0..vpos0+k1-1: library GEMMs
+        """cuda_graph_executor.py:245-268 for the k1 tokens in vtok at vpos0..vpos0+k1-1: solort_gemm_rows
         on the k1 rows around solort_decode_layer (nq = k1: prologue, KV write, causal attention over
         the bucket), the logits [k1, V], their argmax (:475) and the accepted-prefix rule (:476-481)
         into acc_ver = [a, tg[a]]."""
         s, w = self.s, self.w
         ops.rope_rows(self.inv_freq, self.vpos0, self.k1, self.cs_ver)          # :248
         x = w.embed.index_select(0, self.vtok)                                  # :249
-        h = torch.empty_like(x)
-        ops.add_rmsnorm(x, None, w.in_ln[0], self.eps, None, h)                  # :252
+        bf = dict(dtype=torch.bfloat16, device=self.dev)
+        qkv, act = torch.empty(self.k1, s.qkv_width, **bf), torch.empty(self.k1, s.inter, **bf)
+        logits = torch.empty(self.k1, s.vocab, **bf)
         for li in range(s.layers):
-            qkv = F.linear(h, w.wqkv[li])                                        # :253
+            ops.gemm_rows(w.wqkv[li], x, qkv, w.in_ln[li], self.eps)             # :252-253
             ops.decode_layer(qkv, w.qn[li], w.kn[li], self.eps, self.cs_ver, self.vpos0, self.kc[li], self.vc[li],
                              bound, self.scale, self.ws_ver, verify_splits(bound, s.nkv), self.ctx_ver, s.nh, s.nkv)
-            self._mlp_rows(li, x, h, self.ctx_ver)                               # :264-267
-        ops.add_rmsnorm(x, None, w.final_norm, self.eps, None, h)
-        logits = F.linear(h, w.lm_head)                                          # :268
+            ops.gemm_rows(w.wo[li], self.ctx_ver, x, res=x, mode=ops.GEMV_RESID)  # :264
+            ops.gemm_rows(w.wgu[li], x, act, w.post_ln[li], self.eps, mode=ops.GEMV_SWIGLU, inter=s.inter)  # :265-266
+            ops.gemm_rows(w.wd[li], act, x, res=x, mode=ops.GEMV_RESID)          # :267
+        ops.gemm_rows(w.lm_head, x, logits, w.final_norm, self.eps)              # :268
         ops.argmax_rows(logits, self.tok_ver, self.ws_argv)
         if self.k1 > 1:
             ops.accept_prefix(self.tok_ver, self.vtok[1:], self.acc_ver)
@@ -316,7 +318,7 @@ class GraphQwen3Decode:
         bound = verify_bound(pos0 + self.k1 - 1, self.buckets)
         self.vpos0.fill_(int(pos0))
         if bound not in self._ver_graphs:
-            self._verify_forward(bound)  # eager once: the GEMM library initialises outside the capture
+            self._verify_forward(bound)  # eager once, outside the capture
             graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(graph):
                 self._ver_logits[bound] = self._verify_forward(bound)

@@ -605,6 +605,37 @@ def gemv(w: torch.Tensor, x: torch.Tensor, out: torch.Tensor, norm_w: torch.Tens
     _lib.check(rc, "gemv")
 
 
+GEMM_ROWS_MAX = 16
+
+
+def gemm_rows(w: torch.Tensor, x: torch.Tensor, out: torch.Tensor, norm_w: torch.Tensor | None = None,
+              eps: float = 1e-6, res: torch.Tensor | None = None, mode: int = GEMV_PLAIN, inter: int = 0) -> None:
+    """gemv for the rows of x [m, k], m <= GEMM_ROWS_MAX: out [m, n] = x W^T with the same fused neighbours
+    (res [m, n], may be out); see solort_gemm_rows."""
+    _need(x.dim() == 2 and out.dim() == 2 and w.dim() == 2, "w, x and out must be 2-D")
+    m, k = x.shape
+    n = out.shape[1]
+    _need(1 <= m <= GEMM_ROWS_MAX, f"x must have 1..{GEMM_ROWS_MAX} rows (got {m})")
+    _rows("x", x, m, k)
+    _rows("out", out, m, n)
+    _rows("w", w, w.shape[0], k)
+    if mode == GEMV_SWIGLU:
+        _need(inter >= n and w.shape[0] >= inter + n, f"w must hold gate and up rows (inter {inter}, n {n})")
+    else:
+        _need(w.shape[0] >= n, f"w has {w.shape[0]} rows, fewer than n = {n}")
+    if norm_w is not None:
+        _on_gpu("norm_w", norm_w, torch.bfloat16)
+        _need(norm_w.numel() == k and norm_w.is_contiguous(), f"norm_w must hold k = {k} values")
+    if mode == GEMV_RESID:
+        _need(res is not None, "GEMV_RESID needs res")
+        _rows("res", res, m, n)
+    rc = _lib.load().solort_gemm_rows(
+        w.data_ptr(), w.stride(0), n, k, x.data_ptr(), x.stride(0), m, None if norm_w is None else norm_w.data_ptr(),
+        float(eps), None if res is None else res.data_ptr(), 0 if res is None else res.stride(0), int(mode), int(inter),
+        out.data_ptr(), out.stride(0), _stream(w))
+    _lib.check(rc, "gemm_rows")
+
+
 def gemv_argmax_workspace(n_out: int, device: torch.device | str) -> torch.Tensor:
     """Workspace for gemv_argmax over n_out outputs (allocate once, reuse)."""
     nbytes = _lib.load().solort_gemv_argmax_workspace_bytes(int(n_out))
