@@ -372,6 +372,15 @@ int solort_add_rmsnorm(const void* x, int64_t x_row_stride, const void* y, int64
                        solort_stream_t stream);
 
 /*
+ * solort_add_rmsnorm with y given as the fp32 shares parts [n_parts][m][k] of
+ * solort_gemm_tile: x_out = x + bf16(sum of the shares), added in order, then h =
+ * _rmsnorm(x_out, norm_w); norm_w NULL: x_out only (h is not read).  k <= 8192.
+ */
+int solort_add_parts_rmsnorm(const void* x, int64_t x_row_stride, const void* parts, int n_parts, const void* norm_w,
+                             float eps, int m, int k, void* x_out, int64_t x_out_row_stride, void* h,
+                             int64_t h_row_stride, solort_stream_t stream);
+
+/*
  * out[r][i] = silu(gu[r][i]) * gu[r][inter + i] over m gate_up rows
  * (cuda_graph_executor.py:132-134, :265-267), silu and the product each
  * rounded to bf16.  inter and the row strides multiples of 8, 16-byte
@@ -407,6 +416,27 @@ int solort_gemv(const void* w, int64_t w_row_stride, int n_out, int k, const voi
 int solort_gemm_rows(const void* w, int64_t w_row_stride, int n_out, int k, const void* x, int64_t x_row_stride, int m,
                      const void* norm_w, float eps, const void* res, int64_t res_row_stride, int mode, int64_t inter,
                      void* out, int64_t out_row_stride, solort_stream_t stream);
+
+/*
+ * The products of a prompt bucket's rows (cuda_graph_executor.py:115,
+ * :131-134): X [m][x_row_stride] times W^T, W [rows][w_row_stride] bf16
+ * row-major, fp32 accumulation.  mode:
+ *   SOLORT_TILE_PLAIN   out [m][out_row_stride] bf16 = X W^T
+ *   SOLORT_TILE_SWIGLU  out[t][i] = silu(g) * u, g and u the products with rows
+ *                       i and inter + i of W, each rounded to bf16, as silu is
+ *   SOLORT_TILE_PARTS   out [n_parts][m][n_out] fp32: the sums over n_parts
+ *                       contiguous shares of k, for solort_add_parts_rmsnorm
+ *                       (n_parts <= k / 256; solort_gemm_tile_parts(m, n_out,
+ *                       k) gives the count that fills the device, 0 for a
+ *                       shape the product does not take)
+ * n_out a multiple of 4, k a multiple of 128 from 512 to 65536; w, x and out
+ * 16-byte aligned, row strides of w and x multiples of 8, of out 4; w and x
+ * below 2 GiB.  out must not overlap x or w.
+ */
+enum { SOLORT_TILE_PLAIN = 0, SOLORT_TILE_SWIGLU = 1, SOLORT_TILE_PARTS = 2 };
+int solort_gemm_tile_parts(int m, int n_out, int k);
+int solort_gemm_tile(const void* w, int64_t w_row_stride, int n_out, int k, const void* x, int64_t x_row_stride, int m,
+                     int mode, int64_t inter, int n_parts, void* out, int64_t out_row_stride, solort_stream_t stream);
 
 /* Workspace bytes for solort_gemv_argmax with n_out outputs (one 8-byte key
  * per workgroup; no zero-fill needed). */

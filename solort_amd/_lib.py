@@ -101,6 +101,10 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
         c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_float, c_int, c_int, c_void_p, c_int64, c_void_p,
                 c_int64, c_void_p],
     ),
+    "solort_add_parts_rmsnorm": (
+        c_int, [c_void_p, c_int64, c_void_p, c_int, c_void_p, c_float, c_int, c_int, c_void_p, c_int64, c_void_p,
+                c_int64, c_void_p],
+    ),
     "solort_swiglu_rows": (c_int, [c_void_p, c_int64, c_int, c_int, c_void_p, c_int64, c_void_p]),
     "solort_gemv": (
         c_int,
@@ -109,6 +113,11 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "solort_gemm_rows": (
         c_int, [c_void_p, c_int64, c_int, c_int, c_void_p, c_int64, c_int, c_void_p, c_float, c_void_p, c_int64, c_int,
                 c_int64, c_void_p, c_int64, c_void_p],
+    ),
+    "solort_gemm_tile_parts": (c_int, [c_int, c_int, c_int]),
+    "solort_gemm_tile": (
+        c_int, [c_void_p, c_int64, c_int, c_int, c_void_p, c_int64, c_int, c_int, c_int64, c_int, c_void_p, c_int64,
+                c_void_p],
     ),
     "solort_gemv_argmax_workspace_bytes": (c_size_t, [c_int]),
     "solort_gemv_argmax": (

@@ -1,6 +1,7 @@
 // Row-wise neighbours of a multi-row layer (prompt prefill, speculative
 // verify) around the library matrix products, one launch each:
 //   add_rmsnorm  x = x + y (the residual sum), h = _rmsnorm(x, w)
+//   add_parts_rmsnorm  the same with y as fp32 shares of a product split over k
 //   swiglu_rows  act = silu(gate) * up over the two halves of a gate_up row
 //
 // Follows src/solort/model/cuda_graph_executor.py:25-28 (_rmsnorm), :131-135
@@ -103,6 +104,65 @@ __global__ __launch_bounds__(256) void add_rmsnorm_kernel(const uint16_t* x, int
   }
 }
 
+// x_out = x + bf16(sum of the n_parts fp32 shares of y), h = _rmsnorm(x_out, w) (NORM): the end of a product whose
+// k was split over workgroups (solort_gemm_tile).  One workgroup per row, a thread per 16-byte chunk of the row (two
+// from k = 4096 on), so that a row's shares are all in flight at once; the shares are added in order.
+template <bool NORM>
+__global__ __launch_bounds__(512) void add_parts_rmsnorm_kernel(const uint16_t* x, int64_t x_stride,
+                                                                const float* __restrict__ parts, int n_parts,
+                                                                const uint16_t* __restrict__ w, int m, int k, float eps,
+                                                                uint16_t* x_out, int64_t xo_stride,
+                                                                uint16_t* __restrict__ h, int64_t h_stride) {
+  __shared__ float s_red[8];
+  const int64_t row = blockIdx.x;
+  const int tid = threadIdx.x, nch = k >> 3, nw = blockDim.x >> 6;
+  const float* p = parts + row * k;
+  const int64_t part = (int64_t)m * k;
+  float v[2][8];
+  float ss = 0.f;
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int i = tid + (int)blockDim.x * q;
+    if (i >= nch) break;
+    float y[8] = {};
+#pragma unroll 4
+    for (int s = 0; s < n_parts; ++s) {
+      const float4 a = *reinterpret_cast<const float4*>(p + s * part + 8 * i);
+      const float4 b = *reinterpret_cast<const float4*>(p + s * part + 8 * i + 4);
+      y[0] += a.x; y[1] += a.y; y[2] += a.z; y[3] += a.w;
+      y[4] += b.x; y[5] += b.y; y[6] += b.z; y[7] += b.w;
+    }
+    unpack8(*reinterpret_cast<const uint4*>(x + row * x_stride + 8 * i), v[q]);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[q][e] += rbf(y[e]);
+    const uint4 c = pack8(v[q]);
+    *reinterpret_cast<uint4*>(x_out + row * xo_stride + 8 * i) = c;
+    if constexpr (NORM) {
+      unpack8(c, v[q]);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ss = fmaf(v[q][e], v[q][e], ss);
+    }
+  }
+  if constexpr (NORM) {
+    ss = wave_sum(ss);
+    if ((tid & 63) == 0) s_red[tid >> 6] = ss;
+    __syncthreads();
+    float total = 0.f;
+    for (int i = 0; i < nw; ++i) total += s_red[i];
+    const float r = 1.0f / __builtin_sqrtf(total / (float)k + eps);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int i = tid + (int)blockDim.x * q;
+      if (i >= nch) break;
+      float gv[8];
+      unpack8(*reinterpret_cast<const uint4*>(w + 8 * i), gv);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[q][e] = (v[q][e] * r) * gv[e];
+      *reinterpret_cast<uint4*>(h + row * h_stride + 8 * i) = pack8(v[q]);
+    }
+  }
+}
+
 // One 16-byte chunk of the output per thread.
 __global__ __launch_bounds__(256) void swiglu_rows_kernel(const uint16_t* __restrict__ gu, int64_t gu_stride, int m,
                                                           int inter, uint16_t* __restrict__ out, int64_t out_stride) {
@@ -142,6 +202,32 @@ extern "C" int solort_add_rmsnorm(const void* x, int64_t x_row_stride, const voi
     hipLaunchKernelGGL(add_rmsnorm_kernel<false>, dim3(m), dim3(256), 0, (hipStream_t)stream, (const uint16_t*)x,
                        x_row_stride, nullptr, (int64_t)0, (const uint16_t*)norm_w, k, eps, nullptr, (int64_t)0,
                        (uint16_t*)h, h_row_stride);
+  return check_launch(name);
+}
+
+extern "C" int solort_add_parts_rmsnorm(const void* x, int64_t x_row_stride, const void* parts, int n_parts,
+                                        const void* norm_w, float eps, int m, int k, void* x_out,
+                                        int64_t x_out_row_stride, void* h, int64_t h_row_stride,
+                                        solort_stream_t stream) {
+  const char* name = "add_parts_rmsnorm";
+  if (!x || !parts || !x_out || (norm_w && !h)) return set_error(SOLORT_EINVAL, "%s: null pointer", name);
+  if (m < 1 || k < 8 || k % 8 != 0 || k > 8192 || n_parts < 1)
+    return set_error(SOLORT_EINVAL, "%s: bad shape m=%d k=%d n_parts=%d (k a multiple of 8, <= 8192)", name, m, k,
+                     n_parts);
+  if (x_row_stride < k || x_out_row_stride < k || (norm_w && h_row_stride < k) || x_row_stride % 8 ||
+      x_out_row_stride % 8 || (norm_w && h_row_stride % 8))
+    return set_error(SOLORT_EINVAL, "%s: row strides must be multiples of 8, at least k", name);
+  if (!aligned16(x) || !aligned16(parts) || !aligned16(x_out) || (norm_w && (!aligned16(norm_w) || !aligned16(h))))
+    return set_error(SOLORT_EINVAL, "%s: pointers must be 16-byte aligned", name);
+  const int nch = k / 8, per = (nch + 511) / 512, threads = ((nch + per - 1) / per + 63) / 64 * 64;
+  if (norm_w)
+    hipLaunchKernelGGL(add_parts_rmsnorm_kernel<true>, dim3(m), dim3(threads), 0, (hipStream_t)stream,
+                       (const uint16_t*)x, x_row_stride, (const float*)parts, n_parts, (const uint16_t*)norm_w, m, k,
+                       eps, (uint16_t*)x_out, x_out_row_stride, (uint16_t*)h, h_row_stride);
+  else
+    hipLaunchKernelGGL(add_parts_rmsnorm_kernel<false>, dim3(m), dim3(threads), 0, (hipStream_t)stream,
+                       (const uint16_t*)x, x_row_stride, (const float*)parts, n_parts, nullptr, m, k, eps,
+                       (uint16_t*)x_out, x_out_row_stride, nullptr, (int64_t)0);
   return check_launch(name);
 }
 

@@ -75,6 +75,44 @@ class RandomQwen3:
         self.lm_head = self.embed if s.tie_embeddings else rnd(s.vocab, H)
 
 
+# Rows up to which solort_gemm_tile takes the qkv and gate/up products.  Qwen3-4B, us, with the library's product
+# behind: qkv at 256 rows 20.2 (31.4), 512 30.1 (28.0); gate/up with SwiGLU at 256 rows 42 (47.2 and the SwiGLU's 5),
+# at 512 75 (56.7 and 8).  o_proj and down, whose 2560 outputs alone do not fill the chip, take it at every size
+# (1024 rows: 25.4 and 51.5, library 30.8 and 79.3), unless over many rows the fp32 shares themselves are the cost:
+# a Qwen3-0.6B layer, 8 shares of 1024 outputs, 85.2 us at 512 rows and 111.7 at 1024, with the library 80.4 and 101.6
+# (Qwen3-4B, 6 shares at 512 rows: 175.9, with the library 191.9).
+TILE_QKV_MAX = 256
+TILE_GU_MAX = 256
+PARTS_MAX_LONG = 6
+
+
+class _RowBuffers:
+    """Intermediate rows of a prompt bucket's layers, and which kernel takes each product: up to
+    GEMM_ROWS_MAX rows solort_gemm_rows (few), else solort_gemm_tile where its shape and TILE_*_MAX allow
+    (tile_qkv, tile_gu; o_parts and d_parts: the k shares of the o_proj and down products), else the GEMM
+    library."""
+
+    def __init__(self, s: ModelShape, rows: int, dev: torch.device) -> None:
+        bf = dict(dtype=torch.bfloat16, device=dev)
+        self.few = rows <= ops.GEMM_ROWS_MAX
+        self.act = torch.empty(rows, s.inter, **bf)
+        self.tile_qkv = not self.few and rows <= TILE_QKV_MAX and ops.gemm_tile_parts(rows, s.qkv_width, s.hidden) > 0
+        self.tile_gu = not self.few and rows <= TILE_GU_MAX and ops.gemm_tile_parts(rows, s.inter, s.hidden) > 0
+        if self.few or self.tile_qkv:
+            self.qkv = torch.empty(rows, s.qkv_width, **bf)
+        if self.few:
+            return
+        self.h = torch.empty(rows, s.hidden, **bf)
+
+        def parts(k: int) -> torch.Tensor | None:
+            n = ops.gemm_tile_parts(rows, s.hidden, k) if s.hidden <= 8192 else 0
+            if n == 0 or (rows > 256 and n > PARTS_MAX_LONG):
+                return None
+            return torch.empty(n, rows, s.hidden, dtype=torch.float32, device=dev)
+
+        self.o_parts, self.d_parts = parts(s.nh * HD), parts(s.inter)
+
+
 class GraphQwen3Decode:
     """Greedy decode over a runner-owned bf16 KV cache, one captured graph per KV bucket."""
 
@@ -201,19 +239,20 @@ class GraphQwen3Decode:
 
     def _prefill_forward(self, bound: int) -> torch.Tensor:
         """cuda_graph_executor.py:104-135 over pre_tok[:bound] at positions 0..bound-1: the T-row
-        products as library GEMMs (hipBLASLt), the attention block (with the KV write of rows
-        0..bound-1) as solort_prefill_layer, or for short buckets the prologue then
-        solort_prefill_attn.  Returns the last layer's hidden rows [bound, hidden] (the final norm
-        is applied to the one row the lm_head reads)."""
+        products (_qkv_rows, _mlp_rows), the attention block (with the KV write of rows 0..bound-1) as
+        solort_prefill_layer, or for short buckets the prologue then solort_prefill_attn.  Returns the
+        last layer's hidden rows [bound, hidden] (the final norm is applied to the one row the lm_head
+        reads)."""
         s, w = self.s, self.w
         cs = self.cs_pre[: 2 * bound * (HD // 2)].view(2, bound, HD // 2)
         ops.rope_rows(self.inv_freq, self.zero_pos, bound, cs)                  # :111
         x = w.embed.index_select(0, self.pre_tok[:bound])                       # :112
-        h = torch.empty_like(x)
+        b = _RowBuffers(s, bound, self.dev)
         ctx = self.ctx_pre[:bound]
-        ops.add_rmsnorm(x, None, w.in_ln[0], self.eps, None, h)                  # :114
+        if not b.few:
+            ops.add_rmsnorm(x, None, w.in_ln[0], self.eps, None, b.h)            # :114
         for li in range(s.layers):
-            qkv = F.linear(h, w.wqkv[li])                                        # :115
+            qkv = self._qkv_rows(li, x, b)                                       # :115
             if bound >= FUSED_PREFILL_MIN:                                       # :116-130
                 ops.prefill_layer(qkv, w.qn[li], w.kn[li], self.eps, cs, self.kc[li], self.vc[li], self.scale, ctx,
                                   s.nh, s.nkv)
@@ -221,22 +260,48 @@ class GraphQwen3Decode:
                 ops.qknorm_rope_kvwrite_cs(qkv, w.qn[li], w.kn[li], self.eps, cs, None, self.q_pre[:bound],
                                            self.kc[li], self.vc[li], s.nh, s.nkv)
                 ops.prefill_attn(self.q_pre[:bound], self.kc[li], self.vc[li], self.scale, ctx)
-            self._mlp_rows(li, x, h, ctx)                                        # :131-134
+            self._mlp_rows(li, x, b, ctx)                                        # :131-134
         return x
 
-    def _mlp_rows(self, li: int, x: torch.Tensor, h: torch.Tensor, ctx: torch.Tensor) -> None:
+    def _qkv_rows(self, li: int, x: torch.Tensor, b: "_RowBuffers") -> torch.Tensor:
+        """Layer li's qkv rows: of x through its norm (few rows), or of the normalised b.h."""
+        w = self.w
+        if b.few:
+            ops.gemm_rows(w.wqkv[li], x, b.qkv, w.in_ln[li], self.eps)
+            return b.qkv
+        if b.tile_qkv:
+            ops.gemm_tile(w.wqkv[li], b.h, b.qkv)
+            return b.qkv
+        return F.linear(b.h, w.wqkv[li])
+
+    def _mlp_rows(self, li: int, x: torch.Tensor, b: "_RowBuffers", ctx: torch.Tensor) -> None:
         """The rest of layer li for the rows of ctx (cuda_graph_executor.py:131-134): x gains the
-        layer's two residual terms, and h becomes the next layer's normalised input."""
+        layer's two residual terms, and b.h (not with few rows) becomes the next layer's normalised
+        input."""
         s, w = self.s, self.w
-        ops.add_rmsnorm(x, F.linear(ctx, w.wo[li]), w.post_ln[li], self.eps, x, h)
-        gu = F.linear(h, w.wgu[li])
-        act = torch.empty(x.shape[0], s.inter, dtype=torch.bfloat16, device=self.dev)
-        ops.swiglu_rows(gu, act)
-        y = F.linear(act, w.wd[li])
-        if li + 1 < s.layers:
-            ops.add_rmsnorm(x, y, w.in_ln[li + 1], self.eps, x, h)
+        if b.few:
+            ops.gemm_rows(w.wo[li], ctx, x, res=x, mode=ops.GEMV_RESID)
+            ops.gemm_rows(w.wgu[li], x, b.act, w.post_ln[li], self.eps, mode=ops.GEMV_SWIGLU, inter=s.inter)
+            ops.gemm_rows(w.wd[li], b.act, x, res=x, mode=ops.GEMV_RESID)
+            return
+        self._add_product(w.wo[li], ctx, x, b.o_parts, w.post_ln[li], b.h)
+        if b.tile_gu:
+            ops.gemm_tile(w.wgu[li], b.h, b.act, mode=ops.TILE_SWIGLU, inter=s.inter)
         else:
-            x.add_(y)
+            ops.swiglu_rows(F.linear(b.h, w.wgu[li]), b.act)
+        last = li + 1 == s.layers
+        self._add_product(w.wd[li], b.act, x, b.d_parts, None if last else w.in_ln[li + 1], None if last else b.h)
+
+    def _add_product(self, w: torch.Tensor, y: torch.Tensor, x: torch.Tensor, parts: torch.Tensor | None,
+                     norm_w: torch.Tensor | None, h: torch.Tensor | None) -> None:
+        """x += y @ w.T and h = rmsnorm(x, norm_w) (norm_w None: x only); parts: the product's k shares."""
+        if parts is not None:
+            ops.gemm_tile(w, y, parts, mode=ops.TILE_PARTS)
+            ops.add_parts_rmsnorm(x, parts, norm_w, self.eps, x, h)
+        elif norm_w is not None:
+            ops.add_rmsnorm(x, F.linear(y, w), norm_w, self.eps, x, h)
+        else:
+            x.add_(F.linear(y, w))
 
     def prefill(self, ids: torch.Tensor | list[int]) -> None:
         """Graphed bucketed prefill (cuda_graph_executor.py:149-161) of a prompt of plen tokens: pads

@@ -560,6 +560,29 @@ def add_rmsnorm(x: torch.Tensor, y: torch.Tensor | None, norm_w: torch.Tensor, e
     _lib.check(rc, "add_rmsnorm")
 
 
+def add_parts_rmsnorm(x: torch.Tensor, parts: torch.Tensor, norm_w: torch.Tensor | None, eps: float,
+                      x_out: torch.Tensor, h: torch.Tensor | None) -> None:
+    """add_rmsnorm with y as gemm_tile's fp32 shares [n_parts, m, k]: x_out = x + bf16(their sum), h =
+    rmsnorm(x_out, norm_w); norm_w and h None: x_out only.  See solort_add_parts_rmsnorm."""
+    _need(x.dim() == 2, "x must be [m, k]")
+    m, k = x.shape
+    _rows("x", x, m, k)
+    _rows("x_out", x_out, m, k)
+    _on_gpu("parts", parts, torch.float32)
+    _need(parts.dim() == 3 and parts.shape[1:] == (m, k) and parts.is_contiguous(),
+          f"parts must be contiguous [n_parts, {m}, {k}]")
+    _need((norm_w is None) == (h is None), "norm_w and h go together")
+    if norm_w is not None:
+        _rows("h", h, m, k)
+        _on_gpu("norm_w", norm_w, torch.bfloat16)
+        _need(norm_w.numel() == k and norm_w.is_contiguous(), f"norm_w must hold k = {k} values")
+    rc = _lib.load().solort_add_parts_rmsnorm(
+        x.data_ptr(), x.stride(0), parts.data_ptr(), parts.shape[0], None if norm_w is None else norm_w.data_ptr(),
+        float(eps), m, k, x_out.data_ptr(), x_out.stride(0), None if h is None else h.data_ptr(),
+        0 if h is None else h.stride(0), _stream(x))
+    _lib.check(rc, "add_parts_rmsnorm")
+
+
 def swiglu_rows(gu: torch.Tensor, out: torch.Tensor) -> None:
     """out [m, inter] = silu(gu[:, :inter]) * gu[:, inter:], bf16; see solort_swiglu_rows."""
     _need(out.dim() == 2, "out must be [m, inter]")
@@ -634,6 +657,39 @@ def gemm_rows(w: torch.Tensor, x: torch.Tensor, out: torch.Tensor, norm_w: torch
         float(eps), None if res is None else res.data_ptr(), 0 if res is None else res.stride(0), int(mode), int(inter),
         out.data_ptr(), out.stride(0), _stream(w))
     _lib.check(rc, "gemm_rows")
+
+
+TILE_PLAIN, TILE_SWIGLU, TILE_PARTS = 0, 1, 2
+
+
+def gemm_tile_parts(m: int, n: int, k: int) -> int:
+    """The number of k shares gemm_tile's TILE_PARTS should use for x [m, k] and n outputs; 0 for a shape
+    gemm_tile does not take."""
+    return int(_lib.load().solort_gemm_tile_parts(int(m), int(n), int(k)))
+
+
+def gemm_tile(w: torch.Tensor, x: torch.Tensor, out: torch.Tensor, mode: int = TILE_PLAIN, inter: int = 0) -> None:
+    """x [m, k] W^T for a prompt bucket's rows: bf16 out [m, n] (TILE_SWIGLU: silu(gate) * up of rows i and
+    inter + i of w), or with TILE_PARTS out [n_parts, m, n] fp32, the sums over n_parts shares of k that
+    add_parts_rmsnorm adds; see solort_gemm_tile."""
+    _need(x.dim() == 2 and w.dim() == 2, "w and x must be 2-D")
+    m, k = x.shape
+    n = out.shape[-1]
+    _rows("x", x, m, k)
+    _rows("w", w, w.shape[0], k)
+    if mode == TILE_PARTS:
+        _on_gpu("out", out, torch.float32)
+        _need(out.dim() == 3 and out.shape[1] == m and out.is_contiguous(), f"out must be contiguous [n_parts, {m}, n]")
+    else:
+        _rows("out", out, m, n)
+    if mode == TILE_SWIGLU:
+        _need(inter >= n and w.shape[0] >= inter + n, f"w must hold gate and up rows (inter {inter}, n {n})")
+    else:
+        _need(w.shape[0] >= n, f"w has {w.shape[0]} rows, fewer than n = {n}")
+    rc = _lib.load().solort_gemm_tile(
+        w.data_ptr(), w.stride(0), n, k, x.data_ptr(), x.stride(0), m, int(mode), int(inter),
+        out.shape[0] if mode == TILE_PARTS else 1, out.data_ptr(), out.stride(-2), _stream(w))
+    _lib.check(rc, "gemm_tile")
 
 
 def gemv_argmax_workspace(n_out: int, device: torch.device | str) -> torch.Tensor:
