@@ -349,6 +349,23 @@ int solort_prefill_layer(const void* qkv, int64_t qkv_row_stride, int T, int nh,
                          int out_dtype, solort_stream_t stream);
 
 /*
+ * solort_prefill_layer over qkv rows that a record in device memory points to
+ * (32 bytes, 16-byte aligned), so that a captured graph takes a prompt where the
+ * caller has it.  solort_set_qkv_src writes the record on the stream: layer l's
+ * row t starts at qkv + l * layer_stride + t * row_stride (elements, multiples of
+ * 8), t < rows, width elements each.  T is the graph's row count (its cos/sin
+ * table has T rows): K/V rows 0..T-1 are written, those past the record's rows
+ * as those of zero input, and out rows 0..rows-1.  The rows must stay valid until
+ * the replay has run.
+ */
+int solort_set_qkv_src(void* src, const void* qkv, int64_t layer_stride, int64_t row_stride, int64_t rows, int width,
+                       solort_stream_t stream);
+int solort_prefill_layer_src(const void* src, int layer, int T, int nh, int nkv, int hd, const void* qn_w,
+                             const void* kn_w, float eps, const void* rope_cs, void* k_cache, void* v_cache,
+                             int64_t kv_tok_stride, int64_t kv_head_stride, int64_t max_len, float scale, void* out,
+                             int out_dtype, solort_stream_t stream);
+
+/*
  * Greedy speculative acceptance, on the device.  Replaces
  * cuda_graph_executor.py:476, a = int((tg[:k] == draft).cumprod(0).sum()),
  * and picks the token the round appends after the accepted drafts, tg[a]

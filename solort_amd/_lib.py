@@ -97,6 +97,11 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
          c_int64, c_int64, c_int64, c_float, c_void_p, c_int, c_void_p],
     ),
     "solort_accept_prefix": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p]),
+    "solort_set_qkv_src": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int, c_void_p]),
+    "solort_prefill_layer_src": (
+        c_int, [c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p,
+                c_int64, c_int64, c_int64, c_float, c_void_p, c_int, c_void_p],
+    ),
     "solort_add_rmsnorm": (
         c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_float, c_int, c_int, c_void_p, c_int64, c_void_p,
                 c_int64, c_void_p],

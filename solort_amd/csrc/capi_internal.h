@@ -37,9 +37,17 @@ int noalloc_scratch_setup(int dev);
 
 // prologue.hip: QK-RMSNorm + RoPE of the K rows and the cache write of the K
 // and V rows of T tokens at positions 0..T-1 (no q rows), cos/sin from a
-// solort_rope_rows table; arguments already validated.
+// solort_rope_rows table; arguments already validated.  src: qkv points to a
+// QkvSrc and qkv_row_stride is the layer; tokens past its rows are zeros.
 int launch_kv_rows_cs(const void* qkv, int64_t qkv_row_stride, int T, int nh, int nkv, const void* kn_w, float eps,
                       const void* rope_cs, void* k_cache, void* v_cache, int64_t kv_tok_stride, int64_t kv_head_stride,
-                      int64_t max_len, hipStream_t stream);
+                      int64_t max_len, bool src, hipStream_t stream);
+
+// Where a prompt's qkv rows are, in device memory (32 bytes, written by solort_set_qkv_src): kernels of a captured
+// graph read it, so that a replay takes the caller's tensor where it lies.  Strides in elements.
+struct QkvSrc {
+  const uint16_t* qkv;
+  int64_t layer_stride, row_stride, rows;
+};
 
 }  // namespace solort

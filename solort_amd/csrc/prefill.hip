@@ -121,14 +121,25 @@ __device__ __forceinline__ uint2 lds_read_tr16(const uint16_t* p) {
 // [2][T][64] as solort_qknorm_rope_kvwrite_cs would, bit for bit); t_nkv = T |
 // nkv << 24; round = blocks per KV head in one block per CU; out [T][nh * 128]
 // in fp32 (F32) or bf16; qscale = softmax scale * log2(e).
-template <int G, bool F32, bool FUSED>
+template <int G, bool F32, int FUSED>
 __global__ __launch_bounds__(kThreads, 2) void prefill_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
     const uint16_t* __restrict__ qn_w, const uint16_t* __restrict__ rope_cs, int t_nkv, int tok_stride,
     int head_stride, int q_stride, int round, float qscale, float eps, void* __restrict__ out_ptr) {
-  const int T = t_nkv & 0xffffff, nkv = (int)((unsigned)t_nkv >> 24);
+  const int t_rope = t_nkv & 0xffffff, nkv = (int)((unsigned)t_nkv >> 24);
   constexpr int PB = 64 / G;  // positions per block
-  const int nh = nkv * G, n_qtiles = (T + PB - 1) / PB;
+  const int nh = nkv * G, n_qtiles = (t_rope + PB - 1) / PB;
+  // SRC: q is a QkvSrc in device memory and q_stride the layer.  The grid and the cos/sin table cover t_rope rows, of
+  // which the prompt has T; tiles past it have nothing to do.
+  constexpr bool SRC = FUSED == 2;
+  int T = t_rope;
+  int64_t q_row = q_stride;
+  if constexpr (SRC) {
+    const QkvSrc src = *reinterpret_cast<const QkvSrc*>(q);
+    T = (int)(src.rows < t_rope ? src.rows : t_rope);
+    q = src.qkv + q_stride * src.layer_stride;
+    q_row = src.row_stride;
+  }
   __shared__ __align__(16) uint16_t sK[2][kStage * kKStride];
   __shared__ __align__(16) uint16_t sV[2][kStage * kVStride];
 
@@ -141,6 +152,7 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_kernel(
   const int tile = n_qtiles - 1 - rank;  // first round heaviest first; second round lightest first
   SOLORT_STAMP(tid == 0, (int)blockIdx.x, 0);
   const int p0 = tile * PB;
+  if (SRC && p0 >= T) return;
   const int qrow = p0 + (32 * rg + l32) % PB;                // the query row of this lane's scores
   const int pw = p0 + (G == 1 ? 32 * rg : 0);                // this wave's first position
   const int kend_w = min(T, pw + (PB < 32 ? PB : 32));       // keys this wave attends (wave-uniform)
@@ -152,7 +164,7 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_kernel(
   for (int i = 0; i < 4; ++i) {
     const int R = (tid >> 4) + 16 * i;
     const int pos = min(p0 + R % PB, T - 1);
-    qv[i] = *reinterpret_cast<const uint4*>(q + (int64_t)pos * q_stride + (kvh * G + R / PB) * SOLORT_HD +
+    qv[i] = *reinterpret_cast<const uint4*>(q + pos * q_row + (kvh * G + R / PB) * SOLORT_HD +
                                            8 * (tid & 15));
   }
   // FUSED: this lane's weights and cos/sin values of the q rows it stages (row i at position
@@ -165,7 +177,7 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_kernel(
     for (int pp = 0; pp < NP; ++pp) {
       const int pos = min(p0 + ((tid >> 4) + 16 * pp) % PB, T - 1);
       cs4[pp] = *reinterpret_cast<const uint4*>(rope_cs + (int64_t)pos * 64 + (tid & 7) * 8);
-      sn4[pp] = *reinterpret_cast<const uint4*>(rope_cs + ((int64_t)T + pos) * 64 + (tid & 7) * 8);
+      sn4[pp] = *reinterpret_cast<const uint4*>(rope_cs + ((int64_t)t_rope + pos) * 64 + (tid & 7) * 8);
     }
   }
 
@@ -467,8 +479,9 @@ static int check_prefill(const char* name, int T, int nh, int nkv, int hd, const
 }
 
 // The attention launch; q rows at q + pos * q_stride (elements), fused: raw
-// q rows normalised in the kernel.
-static int launch_prefill(const char* name, const void* q, int64_t q_stride, bool fused, const void* qn_w,
+// q rows normalised in the kernel (1), and found through the QkvSrc at q, layer
+// q_stride (2).
+static int launch_prefill(const char* name, const void* q, int64_t q_stride, int fused, const void* qn_w,
                           const void* rope_cs, float eps, int T, int nh, int nkv, const void* k_cache,
                           const void* v_cache, int64_t kv_tok_stride, int64_t kv_head_stride, float scale, void* out,
                           int out_dtype, hipStream_t s) {
@@ -487,23 +500,31 @@ static int launch_prefill(const char* name, const void* q, int64_t q_stride, boo
                      (const uint16_t*)k_cache, (const uint16_t*)v_cache, (const uint16_t*)qn_w,                      \
                      (const uint16_t*)rope_cs, t_nkv, (int)kv_tok_stride, (int)kv_head_stride, (int)q_stride, round, \
                      qscale, eps, out)
-  switch (G * 4 + (f32 ? 2 : 0) + (fused ? 1 : 0)) {
-    case 4: SOLORT_PREFILL_LAUNCH(1, false, false); break;
-    case 5: SOLORT_PREFILL_LAUNCH(1, false, true); break;
-    case 6: SOLORT_PREFILL_LAUNCH(1, true, false); break;
-    case 7: SOLORT_PREFILL_LAUNCH(1, true, true); break;
-    case 8: SOLORT_PREFILL_LAUNCH(2, false, false); break;
-    case 9: SOLORT_PREFILL_LAUNCH(2, false, true); break;
-    case 10: SOLORT_PREFILL_LAUNCH(2, true, false); break;
-    case 11: SOLORT_PREFILL_LAUNCH(2, true, true); break;
-    case 16: SOLORT_PREFILL_LAUNCH(4, false, false); break;
-    case 17: SOLORT_PREFILL_LAUNCH(4, false, true); break;
-    case 18: SOLORT_PREFILL_LAUNCH(4, true, false); break;
-    case 19: SOLORT_PREFILL_LAUNCH(4, true, true); break;
-    case 32: SOLORT_PREFILL_LAUNCH(8, false, false); break;
-    case 33: SOLORT_PREFILL_LAUNCH(8, false, true); break;
-    case 34: SOLORT_PREFILL_LAUNCH(8, true, false); break;
-    case 35: SOLORT_PREFILL_LAUNCH(8, true, true); break;
+  switch (G * 8 + (f32 ? 4 : 0) + fused) {
+    case 8: SOLORT_PREFILL_LAUNCH(1, false, 0); break;
+    case 9: SOLORT_PREFILL_LAUNCH(1, false, 1); break;
+    case 10: SOLORT_PREFILL_LAUNCH(1, false, 2); break;
+    case 12: SOLORT_PREFILL_LAUNCH(1, true, 0); break;
+    case 13: SOLORT_PREFILL_LAUNCH(1, true, 1); break;
+    case 14: SOLORT_PREFILL_LAUNCH(1, true, 2); break;
+    case 16: SOLORT_PREFILL_LAUNCH(2, false, 0); break;
+    case 17: SOLORT_PREFILL_LAUNCH(2, false, 1); break;
+    case 18: SOLORT_PREFILL_LAUNCH(2, false, 2); break;
+    case 20: SOLORT_PREFILL_LAUNCH(2, true, 0); break;
+    case 21: SOLORT_PREFILL_LAUNCH(2, true, 1); break;
+    case 22: SOLORT_PREFILL_LAUNCH(2, true, 2); break;
+    case 32: SOLORT_PREFILL_LAUNCH(4, false, 0); break;
+    case 33: SOLORT_PREFILL_LAUNCH(4, false, 1); break;
+    case 34: SOLORT_PREFILL_LAUNCH(4, false, 2); break;
+    case 36: SOLORT_PREFILL_LAUNCH(4, true, 0); break;
+    case 37: SOLORT_PREFILL_LAUNCH(4, true, 1); break;
+    case 38: SOLORT_PREFILL_LAUNCH(4, true, 2); break;
+    case 64: SOLORT_PREFILL_LAUNCH(8, false, 0); break;
+    case 65: SOLORT_PREFILL_LAUNCH(8, false, 1); break;
+    case 66: SOLORT_PREFILL_LAUNCH(8, false, 2); break;
+    case 68: SOLORT_PREFILL_LAUNCH(8, true, 0); break;
+    case 69: SOLORT_PREFILL_LAUNCH(8, true, 1); break;
+    case 70: SOLORT_PREFILL_LAUNCH(8, true, 2); break;
   }
 #undef SOLORT_PREFILL_LAUNCH
   return check_launch(name);
@@ -520,7 +541,7 @@ extern "C" int solort_prefill_attn(const void* q, int T, int nh, int nkv, int hd
   if (!q) return set_error(SOLORT_EINVAL, "%s: null pointer", name);
   if (!aligned16(q)) return set_error(SOLORT_EINVAL, "%s: pointers must be 16-byte aligned", name);
   if (T == 0) return 0;
-  return launch_prefill(name, q, (int64_t)nh * SOLORT_HD, false, nullptr, nullptr, 0.f, T, nh, nkv, k_cache, v_cache,
+  return launch_prefill(name, q, (int64_t)nh * SOLORT_HD, 0, nullptr, nullptr, 0.f, T, nh, nkv, k_cache, v_cache,
                         kv_tok_stride, kv_head_stride, scale, out, out_dtype, (hipStream_t)stream);
 }
 
@@ -537,10 +558,51 @@ extern "C" int solort_prefill_layer(const void* qkv, int64_t qkv_row_stride, int
   if (rc || T == 0) return rc;
   hipStream_t s = (hipStream_t)stream;
   rc = launch_kv_rows_cs(qkv, qkv_row_stride, T, nh, nkv, kn_w, eps, rope_cs, k_cache, v_cache, kv_tok_stride,
-                         kv_head_stride, max_len, s);
+                         kv_head_stride, max_len, false, s);
   if (rc) return rc;
-  return launch_prefill(name, qkv, qkv_row_stride, true, qn_w, rope_cs, eps, T, nh, nkv, k_cache, v_cache,
+  return launch_prefill(name, qkv, qkv_row_stride, 1, qn_w, rope_cs, eps, T, nh, nkv, k_cache, v_cache,
                         kv_tok_stride, kv_head_stride, scale, out, out_dtype, s);
+}
+
+namespace {
+
+__global__ void set_qkv_src_kernel(QkvSrc* dst, QkvSrc src) { *dst = src; }
+
+}  // namespace
+
+extern "C" int solort_set_qkv_src(void* src, const void* qkv, int64_t layer_stride, int64_t row_stride, int64_t rows,
+                                  int width, solort_stream_t stream) {
+  const char* name = "set_qkv_src";
+  if (!src || !qkv) return set_error(SOLORT_EINVAL, "%s: null pointer", name);
+  if (!aligned16(src) || !aligned16(qkv)) return set_error(SOLORT_EINVAL, "%s: pointers must be 16-byte aligned", name);
+  if (width < 1 || rows < 1 || row_stride < width || row_stride % 8 || layer_stride < 0 || layer_stride % 8)
+    return set_error(SOLORT_EINVAL, "%s: strides must be multiples of 8, a row at least its width", name);
+  hipLaunchKernelGGL(set_qkv_src_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, (QkvSrc*)src,
+                     QkvSrc{(const uint16_t*)qkv, layer_stride, row_stride, rows});
+  return check_launch(name);
+}
+
+// Reading the rows through the record adds a dependent load to each kernel and saves the caller a copy of the prompt's
+// qkv into buffers of its own, and the tiles past a ragged prompt their work: 36 Qwen3-4B layers of 1024 rows in one
+// graph 1056 -> 913 us (a copy of 453 MB).  Below 256 rows the loads cost what the copy does, so short prompts copy.
+extern "C" int solort_prefill_layer_src(const void* src, int layer, int T, int nh, int nkv, int hd, const void* qn_w,
+                                        const void* kn_w, float eps, const void* rope_cs, void* k_cache, void* v_cache,
+                                        int64_t kv_tok_stride, int64_t kv_head_stride, int64_t max_len, float scale,
+                                        void* out, int out_dtype, solort_stream_t stream) {
+  const char* name = "prefill_layer_src";
+  if (layer < 0) return set_error(SOLORT_EINVAL, "%s: layer %d", name, layer);
+  const int64_t width = (int64_t)(nh + 2 * nkv) * hd;  // the row stride was checked when the record was written
+  int rc = check_prologue(name, src, width, T, nh, nkv, hd, qn_w, kn_w, rope_cs, out, k_cache, v_cache, kv_tok_stride,
+                          kv_head_stride, max_len);
+  if (rc) return rc;
+  rc = check_prefill(name, T, nh, nkv, hd, k_cache, v_cache, kv_tok_stride, kv_head_stride, max_len, out, out_dtype);
+  if (rc || T == 0) return rc;
+  hipStream_t s = (hipStream_t)stream;
+  rc = launch_kv_rows_cs(src, layer, T, nh, nkv, kn_w, eps, rope_cs, k_cache, v_cache, kv_tok_stride, kv_head_stride,
+                         max_len, true, s);
+  if (rc) return rc;
+  return launch_prefill(name, src, layer, 2, qn_w, rope_cs, eps, T, nh, nkv, k_cache, v_cache, kv_tok_stride,
+                        kv_head_stride, scale, out, out_dtype, s);
 }
 
 #ifdef SOLORT_PHASE_STAMPS

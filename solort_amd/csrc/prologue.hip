@@ -22,7 +22,9 @@ namespace solort {
 // rope_src: TABLE, the step's cos/sin rows rope_cs [2][T][64] bf16; else
 // inv_freq [64] fp32.  The arguments the first loads need lead (qkv ..
 // rope_src: 14 dwords), so they arrive preloaded in SGPRs.
-template <bool TABLE>
+// SRC: qkv is a QkvSrc in device memory and qkv_stride the layer; rows past
+// the prompt's are zeros.
+template <bool TABLE, bool SRC>
 __global__ __launch_bounds__(256) void qknorm_rope_kvwrite_kernel(
     const uint16_t* __restrict__ qkv, int64_t qkv_stride, int T, int nh, int nkv, int row0,
     const uint16_t* __restrict__ qn_w, const uint16_t* __restrict__ kn_w, const void* __restrict__ rope_src,
@@ -46,10 +48,17 @@ __global__ __launch_bounds__(256) void qknorm_rope_kvwrite_kernel(
     sn_raw = *reinterpret_cast<const uint4*>(rope_cs + ((int64_t)T + t) * 64 + (j & 7) * 8);
   }
   const uint4 wq = *reinterpret_cast<const uint4*>(qn_w + j * 8), wk = *reinterpret_cast<const uint4*>(kn_w + j * 8);
-  uint4 raws[kMaxPass];
+  bool live = true;
+  if constexpr (SRC) {
+    const QkvSrc src = *reinterpret_cast<const QkvSrc*>(qkv);
+    live = t < src.rows;
+    qkv = src.qkv + qkv_stride * src.layer_stride;
+    qkv_stride = src.row_stride;
+  }
+  uint4 raws[kMaxPass] = {};
 #pragma unroll
   for (int p = 0; p < kMaxPass; ++p)
-    raws[p] = *reinterpret_cast<const uint4*>(qkv + (int64_t)t * qkv_stride +
+    if (!SRC || live) raws[p] = *reinterpret_cast<const uint4*>(qkv + (int64_t)t * qkv_stride +
                                               min(row0 + slot + 16 * p, heads - 1) * SOLORT_HD + j * 8);
   __builtin_amdgcn_sched_barrier(0);
 
@@ -126,7 +135,7 @@ extern "C" int solort_qknorm_rope_kvwrite(const void* qkv, int64_t qkv_row_strid
   int rc = check_prologue("qknorm_rope_kvwrite", qkv, qkv_row_stride, T, nh, nkv, hd, qn_w, kn_w, inv_freq, q_out,
                           k_cache, v_cache, kv_tok_stride, kv_head_stride, max_len);
   if (rc || T == 0) return rc;
-  hipLaunchKernelGGL(qknorm_rope_kvwrite_kernel<false>, dim3((unsigned)T), dim3(256), 0, (hipStream_t)stream,
+  hipLaunchKernelGGL((qknorm_rope_kvwrite_kernel<false, false>), dim3((unsigned)T), dim3(256), 0, (hipStream_t)stream,
                      (const uint16_t*)qkv, qkv_row_stride, T, nh, nkv, 0, (const uint16_t*)qn_w,
                      (const uint16_t*)kn_w, (const void*)inv_freq, eps, max_len, pos0_dev, (uint16_t*)q_out,
                      (uint16_t*)k_cache, (uint16_t*)v_cache, kv_tok_stride, kv_head_stride);
@@ -141,7 +150,7 @@ extern "C" int solort_qknorm_rope_kvwrite_cs(const void* qkv, int64_t qkv_row_st
   int rc = check_prologue("qknorm_rope_kvwrite_cs", qkv, qkv_row_stride, T, nh, nkv, hd, qn_w, kn_w, rope_cs,
                           q_out, k_cache, v_cache, kv_tok_stride, kv_head_stride, max_len);
   if (rc || T == 0) return rc;
-  hipLaunchKernelGGL(qknorm_rope_kvwrite_kernel<true>, dim3((unsigned)T), dim3(256), 0, (hipStream_t)stream,
+  hipLaunchKernelGGL((qknorm_rope_kvwrite_kernel<true, false>), dim3((unsigned)T), dim3(256), 0, (hipStream_t)stream,
                      (const uint16_t*)qkv, qkv_row_stride, T, nh, nkv, 0, (const uint16_t*)qn_w,
                      (const uint16_t*)kn_w, rope_cs, eps, max_len, pos0_dev, (uint16_t*)q_out, (uint16_t*)k_cache,
                      (uint16_t*)v_cache, kv_tok_stride, kv_head_stride);
@@ -151,12 +160,17 @@ extern "C" int solort_qknorm_rope_kvwrite_cs(const void* qkv, int64_t qkv_row_st
 // The K and V rows of T tokens at positions 0..T-1 (the prefill layer's
 // prologue; its q rows are normalised inside the attention kernel).  The
 // caller has validated the arguments as for solort_qknorm_rope_kvwrite_cs.
+// src: qkv is a QkvSrc in device memory and qkv_row_stride the layer.
 int solort::launch_kv_rows_cs(const void* qkv, int64_t qkv_row_stride, int T, int nh, int nkv, const void* kn_w,
                               float eps, const void* rope_cs, void* k_cache, void* v_cache, int64_t kv_tok_stride,
-                              int64_t kv_head_stride, int64_t max_len, hipStream_t stream) {
-  hipLaunchKernelGGL(qknorm_rope_kvwrite_kernel<true>, dim3((unsigned)T), dim3(256), 0, stream, (const uint16_t*)qkv,
-                     qkv_row_stride, T, nh, nkv, nh, (const uint16_t*)kn_w, (const uint16_t*)kn_w, rope_cs, eps,
-                     max_len, (const int64_t*)nullptr, (uint16_t*)nullptr, (uint16_t*)k_cache, (uint16_t*)v_cache,
-                     kv_tok_stride, kv_head_stride);
+                              int64_t kv_head_stride, int64_t max_len, bool src, hipStream_t stream) {
+#define SOLORT_KV_ROWS(SS)                                                                                           \
+  hipLaunchKernelGGL((qknorm_rope_kvwrite_kernel<true, SS>), dim3((unsigned)T), dim3(256), 0, stream,                  \
+                     (const uint16_t*)qkv, qkv_row_stride, T, nh, nkv, nh, (const uint16_t*)kn_w,                      \
+                     (const uint16_t*)kn_w, rope_cs, eps, max_len, (const int64_t*)nullptr, (uint16_t*)nullptr,        \
+                     (uint16_t*)k_cache, (uint16_t*)v_cache, kv_tok_stride, kv_head_stride)
+  if (src) SOLORT_KV_ROWS(true);
+  else SOLORT_KV_ROWS(false);
+#undef SOLORT_KV_ROWS
   return check_launch("prefill_layer (K/V rows)");
 }

@@ -436,16 +436,10 @@ def prefill_attn(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, 
     _lib.check(rc, "prefill_attn")
 
 
-def prefill_layer(qkv: torch.Tensor, qn_w: torch.Tensor, kn_w: torch.Tensor, eps: float, rope_cs: torch.Tensor,
-                  k_cache: torch.Tensor, v_cache: torch.Tensor, scale: float, out: torch.Tensor, nh: int,
-                  nkv: int) -> None:
-    """One layer's prefill attention block for T prompt rows at positions 0..T-1: qkv
-    [T, (nh+2nkv)*128] -> K/V cache rows 0..T-1 and out [T, nh*128]; rope_cs = rope_rows(inv_f,
-    0, T).  Equal, bit for bit, to qknorm_rope_kvwrite_cs + prefill_attn; see solort_prefill_layer."""
-    _on_gpu("qkv", qkv, torch.bfloat16)
-    _need(qkv.dim() == 2 and qkv.shape[1] == (nh + 2 * nkv) * HD and qkv.stride(1) == 1,
-          f"qkv must be [T, {(nh + 2 * nkv) * HD}] with unit column stride")
-    T = qkv.shape[0]
+def _prefill_layer_args(T: int, qn_w: torch.Tensor, kn_w: torch.Tensor, rope_cs: torch.Tensor,
+                        k_cache: torch.Tensor, v_cache: torch.Tensor, out: torch.Tensor, nh: int,
+                        nkv: int) -> tuple[int, int, int, int]:
+    """Checks what the prefill layer calls share; (KV token stride, head stride, max_len, output type)."""
     for name, w in (("qn_w", qn_w), ("kn_w", kn_w)):
         _on_gpu(name, w, torch.bfloat16)
         _need(w.shape == (HD,) and w.is_contiguous(), f"{name} must be [{HD}] contiguous")
@@ -458,11 +452,64 @@ def prefill_layer(qkv: torch.Tensor, qn_w: torch.Tensor, kn_w: torch.Tensor, eps
     _need(out.shape == (T, nh * HD) and out.is_contiguous() and out.data_ptr() % 16 == 0,
           f"out must be [{T}, {nh * HD}] contiguous and 16-byte aligned")
     dt = DTYPE_F32 if out.dtype == torch.float32 else DTYPE_BF16
+    return ts, hs, max_len, dt
+
+
+def prefill_layer(qkv: torch.Tensor, qn_w: torch.Tensor, kn_w: torch.Tensor, eps: float, rope_cs: torch.Tensor,
+                  k_cache: torch.Tensor, v_cache: torch.Tensor, scale: float, out: torch.Tensor, nh: int,
+                  nkv: int) -> None:
+    """One layer's prefill attention block for T prompt rows at positions 0..T-1: qkv
+    [T, (nh+2nkv)*128] -> K/V cache rows 0..T-1 and out [T, nh*128]; rope_cs = rope_rows(inv_f,
+    0, T).  Equal, bit for bit, to qknorm_rope_kvwrite_cs + prefill_attn; see solort_prefill_layer."""
+    _on_gpu("qkv", qkv, torch.bfloat16)
+    _need(qkv.dim() == 2 and qkv.shape[1] == (nh + 2 * nkv) * HD and qkv.stride(1) == 1,
+          f"qkv must be [T, {(nh + 2 * nkv) * HD}] with unit column stride")
+    T = qkv.shape[0]
+    ts, hs, max_len, dt = _prefill_layer_args(T, qn_w, kn_w, rope_cs, k_cache, v_cache, out, nh, nkv)
     rc = _lib.load().solort_prefill_layer(
         qkv.data_ptr(), qkv.stride(0), T, nh, nkv, HD, qn_w.data_ptr(), kn_w.data_ptr(), float(eps),
         rope_cs.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), ts, hs, max_len, float(scale), out.data_ptr(), dt,
         _stream(qkv))
     _lib.check(rc, "prefill_layer")
+
+
+def qkv_src(device: torch.device | str) -> torch.Tensor:
+    """A record for set_qkv_src and prefill_layer_src."""
+    return torch.zeros(4, dtype=torch.int64, device=device)
+
+
+def qkv_src_takes(qkv: torch.Tensor, device: torch.device) -> bool:
+    """Whether set_qkv_src can point to qkv [layers, rows, width] where it lies."""
+    return (qkv.device == device and qkv.dtype == torch.bfloat16 and qkv.dim() == 3 and qkv.stride(2) == 1
+            and qkv.data_ptr() % 16 == 0 and qkv.stride(0) % 8 == 0 and qkv.stride(1) % 8 == 0
+            and qkv.stride(1) >= qkv.shape[2] and qkv.shape[1] > 0)
+
+
+def set_qkv_src(src: torch.Tensor, qkv: torch.Tensor) -> None:
+    """Points the record at the rows of qkv [layers, rows, width]; see solort_set_qkv_src."""
+    _on_gpu("src", src, torch.int64)
+    _need(src.shape == (4,) and src.is_contiguous(), "src must be a qkv_src record")
+    _on_gpu("qkv", qkv, torch.bfloat16)
+    _need(qkv_src_takes(qkv, src.device), "qkv must be [layers, rows, width] bf16 rows, strides multiples of 8")
+    rc = _lib.load().solort_set_qkv_src(src.data_ptr(), qkv.data_ptr(), qkv.stride(0), qkv.stride(1), qkv.shape[1],
+                                        qkv.shape[2], _stream(src))
+    _lib.check(rc, "set_qkv_src")
+
+
+def prefill_layer_src(src: torch.Tensor, layer: int, qn_w: torch.Tensor, kn_w: torch.Tensor, eps: float,
+                      rope_cs: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, scale: float,
+                      out: torch.Tensor, nh: int, nkv: int) -> None:
+    """prefill_layer over the rows the record points to: cache rows 0..T-1 (T rows of out and rope_cs; past the
+    record's rows those of zero input) and the record's rows of out.  The record's qkv must be as wide as nh and
+    nkv say; see solort_prefill_layer_src."""
+    _on_gpu("src", src, torch.int64)
+    _need(src.shape == (4,) and src.is_contiguous(), "src must be a qkv_src record")
+    T = out.shape[0]
+    ts, hs, max_len, dt = _prefill_layer_args(T, qn_w, kn_w, rope_cs, k_cache, v_cache, out, nh, nkv)
+    rc = _lib.load().solort_prefill_layer_src(
+        src.data_ptr(), int(layer), T, nh, nkv, HD, qn_w.data_ptr(), kn_w.data_ptr(), float(eps), rope_cs.data_ptr(),
+        k_cache.data_ptr(), v_cache.data_ptr(), ts, hs, max_len, float(scale), out.data_ptr(), dt, _stream(src))
+    _lib.check(rc, "prefill_layer_src")
 
 
 def argmax_workspace(rows: int, device: torch.device | str) -> torch.Tensor:

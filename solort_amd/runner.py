@@ -149,6 +149,7 @@ class GraphQwen3Attention:
         # prefill: padded prompt rows per layer, bucketed graphs
         pmax = self.pre_buckets[-1]
         self.qkv_pre = torch.zeros(layers, pmax, self.width, dtype=torch.bfloat16, device=self.dev)
+        self.src_pre = ops.qkv_src(self.dev)  # where the fused layers' graph finds the prompt's qkv rows
         self.zero_pos = torch.zeros(1, dtype=torch.long, device=self.dev)  # prefill positions start at 0
         self.cs_pre = torch.zeros(2 * pmax * (HD // 2), dtype=torch.bfloat16, device=self.dev)  # step cos/sin
         self.ctx_pre = torch.zeros(layers, pmax, nh * HD, dtype=torch.bfloat16, device=self.dev)
@@ -210,25 +211,38 @@ class GraphQwen3Attention:
         ops.rope_rows(self.inv_freq, self.zero_pos, bound, cs)  # cos/sin once per step (:111)
         for li in range(self.L):
             if bound >= FUSED_PREFILL_MIN:  # prologue of the K/V rows, then attention normalising q itself
-                ops.prefill_layer(self.qkv_pre[li, :bound], self.qn_w[li], self.kn_w[li], self.eps, cs, self.kc[li],
-                                  self.vc[li], self.scale, self.ctx_pre[li, :bound], self.nh, self.nkv)
+                ops.prefill_layer_src(self.src_pre, li, self.qn_w[li], self.kn_w[li], self.eps, cs, self.kc[li],
+                                      self.vc[li], self.scale, self.ctx_pre[li, :bound], self.nh, self.nkv)
             else:  # short prompts: the whole prologue, then attention on the materialised q
                 ops.qknorm_rope_kvwrite_cs(self.qkv_pre[li, :bound], self.qn_w[li], self.kn_w[li], self.eps, cs,
                                            None, self.q_pre[:bound], self.kc[li], self.vc[li], self.nh, self.nkv)
                 ops.prefill_attn(self.q_pre[:bound], self.kc[li], self.vc[li], self.scale,
                                  self.ctx_pre[li, :bound])
 
+    def _rows_fit(self, qkv: torch.Tensor) -> bool:
+        """Whether a replay can read qkv where it lies: the shape copy_ would take without broadcasting, as bf16 rows
+        on this device."""
+        return (qkv.dim() == 3 and qkv.shape[0] == self.L and qkv.shape[2] == self.width
+                and ops.qkv_src_takes(qkv, self.kc.device))
+
     def prefill(self, qkv: torch.Tensor) -> torch.Tensor:
         """Graphed bucketed prefill (cuda_graph_executor.py:149-161): qkv [layers, plen, width] for
-        prompt positions 0..plen-1, padded with zero rows to the first bucket >= plen.  Writes cache
+        prompt positions 0..plen-1, padded with zero rows to the first bucket >= plen (from
+        FUSED_PREFILL_MIN on without a copy: the replay reads the rows of qkv itself).  Writes cache
         rows 0..bucket-1 (padding rows included, as in the reference; decode never reads them) and
         returns ctx [layers, plen, nh*128] (a view of the static buffer)."""
         plen = int(qkv.shape[1])
         bound = next((b for b in self.pre_buckets if b >= plen), None)
         if bound is None or plen < 1:
             raise RuntimeError(f"prompt length {plen} outside the prefill buckets {self.pre_buckets}")
-        self.qkv_pre[:, :plen].copy_(qkv)
-        self.qkv_pre[:, plen:bound].zero_()
+        if bound >= FUSED_PREFILL_MIN and self._rows_fit(qkv):
+            ops.set_qkv_src(self.src_pre, qkv)  # the replay reads the caller's rows
+            qkv.record_stream(torch.cuda.current_stream(qkv.device))
+        else:
+            self.qkv_pre[:, :plen].copy_(qkv)
+            self.qkv_pre[:, plen:bound].zero_()
+            if bound >= FUSED_PREFILL_MIN:
+                ops.set_qkv_src(self.src_pre, self.qkv_pre[:, :plen])
         if bound not in self._pre_graphs:
             graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(graph):
