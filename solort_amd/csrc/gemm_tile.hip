@@ -16,7 +16,7 @@
 // barrier a stage.  Each stage buffer is an array of its own: the compiler then
 // sees that a stage's reads do not touch the buffers being filled and adds no
 // full wait.  A row's 16-byte chunks are stored in the order chunk ^ (row %
-// chunks), by permuting the lanes' source addresses, so the 16 rows of an
+// chunks) (rows of four chunks: row / 2), by permuting the lanes' source addresses, so the 16 rows of an
 // operand read fall on different banks.
 // A CU sustains about 35 GB/s of such loads whatever their depth, so the tile is
 // chosen to give every CU one workgroup and few repeated reads of X (launches of
@@ -26,7 +26,7 @@
 // Measured on MI355X, Qwen3-4B widths, graphs over 10 weight copies, 32 / 128 /
 // 1024 rows, the library's product behind (us): qkv 10.0 / 16.6 / - (11.7 / 19.1
 // / 38.1), o_proj 5.8 / 7.8 / 25.4 (9.3 / 19.3 / 30.8), gate_up with SwiGLU 21.7
-// / 32.1 / - (24.6 / 31.2 / 106.5 without), down 11.8 / 17.7 / 51.5 (21.4 / 52.6
+// / 32.1 / 102 (24.6 / 31.2 / 106.5 without), down 11.8 / 17.7 / 51.5 (21.4 / 52.6
 // / 79.3).
 #include "common.h"
 #include "capi_internal.h"
@@ -66,8 +66,9 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(
     int inter, void* __restrict__ out_ptr, int64_t out_stride) {
   constexpr int NW = WM * WN, MT = BM / WM / 16, NT = BN / WN / 16;
   constexpr int ROWS = BM + BN, KC = kBK / 8, RPI = 64 / KC,
-                IPW = ROWS / RPI / NW;  // load instructions per wavefront and stage
-  static_assert(ROWS % (RPI * NW) == 0 && BM % RPI == 0 && BM % (16 * WM) == 0 && BN % (16 * WN) == 0, "tile shape");
+                NI = ROWS / RPI, IPW = (NI + NW - 1) / NW;  // load instructions per wavefront and stage
+  constexpr int KS = KC == 4 ? 1 : 0;  // rows of four chunks: two rows fill a bank period
+  static_assert(ROWS % RPI == 0 && BM % RPI == 0 && BM % (16 * WM) == 0 && BN % (16 * WN) == 0, "tile shape");
   static_assert(EPI != kTileSwiglu || NT % 2 == 0, "gate and up blocks of a column meet in one wavefront");
   constexpr int BO = EPI == kTileSwiglu ? BN / 2 : BN;  // outputs per tile
   constexpr int WORDS = ROWS * kBK;
@@ -86,10 +87,12 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(
   };
   const __amdgpu_buffer_rsrc_t xr = rsrc(x, m, x_stride);
   const __amdgpu_buffer_rsrc_t wr = rsrc(w, EPI == kTileSwiglu ? inter + n_out : n_out, w_stride);
+  // First row of this wavefront's j-th load; past the tile's last one it repeats that (the same bytes to the same place).
+  const auto row_of = [&](int j) { return RPI * min(wave + NW * j, NI - 1); };
   int voff[IPW];
 #pragma unroll
   for (int j = 0; j < IPW; ++j) {
-    const int row0 = RPI * (wave + NW * j), row = row0 + lane / KC, ch = (lane ^ row) & (KC - 1);
+    const int row0 = row_of(j), row = row0 + lane / KC, ch = (lane ^ (row >> KS)) & (KC - 1);
     int64_t off;
     if (row0 < BM) {
       off = (int64_t)min(tm * BM + row, m - 1) * x_stride;
@@ -107,7 +110,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(
     const int soff = (k_beg + step) * (kBK * 2);
 #pragma unroll
     for (int j = 0; j < IPW; ++j) {
-      const int row0 = RPI * (wave + NW * j);
+      const int row0 = row_of(j);
       lds_void* dst = (lds_void*)(__attribute__((address_space(3))) uint16_t*)(s + row0 * kBK);
       lds_load16(row0 < BM ? xr : wr, dst, voff[j], soff);
     }
@@ -115,7 +118,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(
   const int r = lane & 15, g = lane >> 4;
   const int wm = wave % WM, wn = wave / WM;
   // chunk 4 kk + g of row r sits in slot (4 kk + g) ^ (r % 8)
-  const int frag = r * kBK + 8 * (g ^ (r & (KC - 1)));
+  const int frag = r * kBK + 8 * (g ^ ((r >> KS) & (KC - 1)));
   const int xbase = wm * (BM / WM) * kBK + frag, wbase = (BM + wn * (BN / WN)) * kBK + frag;
   f32x4_t acc[NT][MT] = {};
   auto compute = [&](const uint16_t* s) {
@@ -280,6 +283,10 @@ extern "C" int solort_gemm_tile(const void* w, int64_t w_row_stride, int n_out, 
     } else if (m <= 128) {
       if (wide) SOLORT_TILE(128, 96, 4, 1, 4, 64, kTileSwiglu);
       else SOLORT_TILE(128, 32, 4, 1, 3, 128, kTileSwiglu);
+    } else if (m > 256) {
+      // 256 rows x 160 outputs, the widest that fits: 1024 rows of N = 9728 are 244 workgroups, one round (102 us; 119
+      // with 64 outputs, library and SwiGLU 117).
+      SOLORT_TILE(256, 320, 4, 2, 3, 32, kTileSwiglu);
     } else {
       if (wide) SOLORT_TILE(256, 96, 4, 1, 3, 64, kTileSwiglu);
       else SOLORT_TILE(128, 64, 4, 2, 3, 128, kTileSwiglu);

@@ -45,7 +45,8 @@ def test_gemm_tile_plain_and_parts(gpu, m, n, k):
 
 
 @pytest.mark.parametrize("m,n,inter,k", [(17, 20, 24, 512), (64, 3072, 3072, 1024), (128, 9728, 9728, 512), (32, 9728, 9728, 512),
-                                         (50, 6200, 6208, 640), (100, 52, 52, 768), (200, 6148, 6160, 512), (300, 40, 40, 640)])
+                                         (50, 6200, 6208, 640), (100, 52, 52, 768), (200, 6148, 6160, 512), (300, 40, 40, 640),
+                                         (1000, 164, 168, 896), (513, 480, 480, 512)])
 def test_gemm_tile_swiglu(gpu, m, n, inter, k):
     print(f"[gemm_tile swiglu m={m} n={n} k={k}]", flush=True)
     x, w = _inputs(m, inter + n, k)
