@@ -493,6 +493,15 @@ int solort_greedy_advance(const void* ws, int vocab, const void* embed, int64_t 
                           void* x, int64_t* tok, int64_t* tokens, int max_tokens, int64_t* step, int64_t* pos,
                           solort_stream_t stream);
 
+/*
+ * The state a greedy chunk starts from, in one launch: *step = 0, *pos =
+ * position, and with x non-NULL *tok = token and x [hidden] = embed row token
+ * (cuda_graph_executor.py:165, :362-374).  Buffers as in solort_greedy_advance;
+ * a token outside [0, vocab) is refused.
+ */
+int solort_decode_start(int64_t token, int64_t position, const void* embed, int vocab, int64_t embed_row_stride,
+                        int hidden, void* x, int64_t* tok, int64_t* step, int64_t* pos, solort_stream_t stream);
+
 /* Workspace bytes for solort_argmax_rows with `rows` rows: per row 64 slots
  * of 16 bytes, then a 16-byte item whose first 32-bit word is the row's
  * epoch (the launch count of the row, which tags the slots each launch

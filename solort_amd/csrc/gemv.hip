@@ -220,6 +220,24 @@ __global__ __launch_bounds__(1024) void greedy_advance_kernel(const uint64_t* __
   }
 }
 
+// The state a greedy chunk starts from: one launch ahead of the replay instead of four tensor ops (three fills and a
+// row gather).  One token of 8 Qwen3-4B layers, host call to host result, 541 -> 533 us.
+__global__ __launch_bounds__(256) void decode_start_kernel(int64_t token, int64_t position,
+                                                           const uint16_t* __restrict__ embed, int64_t row_stride,
+                                                           int hidden, uint16_t* __restrict__ x,
+                                                           int64_t* __restrict__ tok, int64_t* __restrict__ step,
+                                                           int64_t* __restrict__ pos) {
+  if (x) {
+    const uint4* src = reinterpret_cast<const uint4*>(embed + token * row_stride);
+    for (int i = threadIdx.x; i < hidden / 8; i += 256) reinterpret_cast<uint4*>(x)[i] = src[i];
+  }
+  if (threadIdx.x == 0) {
+    if (x) *tok = token;
+    *step = 0;
+    *pos = position;
+  }
+}
+
 }  // namespace solort
 
 using namespace solort;
@@ -351,5 +369,25 @@ extern "C" int solort_greedy_advance(const void* ws, int vocab, const void* embe
   hipLaunchKernelGGL(greedy_advance_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, (const uint64_t*)ws, nkeys,
                      vocab, (const uint16_t*)embed, embed_row_stride, hidden, (uint16_t*)x, tok, tokens, max_tokens, step,
                      pos);
+  return check_launch(name);
+}
+
+extern "C" int solort_decode_start(int64_t token, int64_t position, const void* embed, int vocab,
+                                   int64_t embed_row_stride, int hidden, void* x, int64_t* tok, int64_t* step,
+                                   int64_t* pos, solort_stream_t stream) {
+  const char* name = "decode_start";
+  if (!step || !pos || (x && (!embed || !tok))) return set_error(SOLORT_EINVAL, "%s: null pointer", name);
+  if (((uintptr_t)step & 7u) || ((uintptr_t)pos & 7u)) return set_error(SOLORT_EINVAL, "%s: misaligned buffer", name);
+  if (x) {
+    if (vocab < 1 || hidden < 8 || hidden % 8 != 0 || embed_row_stride < hidden || embed_row_stride % 8 != 0)
+      return set_error(SOLORT_EINVAL, "%s: bad shape vocab=%d hidden=%d stride=%lld", name, vocab, hidden,
+                       (long long)embed_row_stride);
+    if (token < 0 || token >= vocab)
+      return set_error(SOLORT_EINVAL, "%s: token %lld outside the vocabulary %d", name, (long long)token, vocab);
+    if (!aligned16(embed) || !aligned16(x) || ((uintptr_t)tok & 7u))
+      return set_error(SOLORT_EINVAL, "%s: embed and x must be 16-byte, the int64 buffers 8-byte aligned", name);
+  }
+  hipLaunchKernelGGL(decode_start_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, token, position,
+                     (const uint16_t*)embed, embed_row_stride, hidden, (uint16_t*)x, tok, step, pos);
   return check_launch(name);
 }

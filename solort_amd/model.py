@@ -186,10 +186,7 @@ class GraphQwen3Decode:
 
     def start(self, token: int, pos: int) -> None:
         """The first input: token at position pos (rows 0..pos-1 of the cache hold the context)."""
-        self.tok.fill_(int(token))
-        self.pos.fill_(int(pos))
-        self.step.zero_()
-        torch.index_select(self.w.embed, 0, self.tok, out=self.x)     # :165 for the first step
+        ops.decode_start(self.step, self.pos, pos, token, self.w.embed, self.x.view(-1), self.tok)  # with :165
 
     def _step(self, bound: int) -> None:
         """One token: cuda_graph_executor.py:163-190 from the x the previous step (or start) left,
@@ -319,8 +316,11 @@ class GraphQwen3Decode:
         bound = next((b for b in self.pre_buckets if b >= plen), None)
         if bound is None or plen < 1:
             raise RuntimeError(f"prompt length {plen} outside the prefill buckets {self.pre_buckets}")
-        self.pre_tok[:plen].copy_(ids.to(self.dev))
-        self.pre_tok[plen:bound].zero_()
+        if ids.is_cuda:
+            self.pre_tok[:plen].copy_(ids)
+            self.pre_tok[plen:bound].zero_()
+        else:  # the padded prompt in one transfer
+            self.pre_tok[:bound].copy_(F.pad(ids, (0, bound - plen)))
         if bound not in self._pre_graphs:
             self._prefill_forward(bound)  # eager once: the GEMM library initialises outside the capture
             graph = torch.cuda.CUDAGraph()
@@ -330,8 +330,7 @@ class GraphQwen3Decode:
         self._pre_graphs[bound].replay()
         s, w = self.s, self.w
         last = self._pre_hidden[bound][plen - 1]
-        self.pos.fill_(plen - 1)
-        self.step.zero_()
+        ops.decode_start(self.step, self.pos, plen - 1)
         if self.fused_tail:
             ops.gemv_argmax(w.lm_head, last, None, self.ws_arg, w.final_norm, self.eps, logits=self.logits.view(-1))
             ops.greedy_advance(self.ws_arg, s.vocab, w.embed, self.x.view(-1), self.tok, self.tokens, self.step,

@@ -777,6 +777,29 @@ def gemv_argmax(w: torch.Tensor, x: torch.Tensor, out_idx: torch.Tensor | None, 
     _lib.check(rc, "gemv_argmax")
 
 
+def decode_start(step: torch.Tensor, pos: torch.Tensor, position: int, token: int = 0,
+                 embed: torch.Tensor | None = None, x: torch.Tensor | None = None,
+                 tok: torch.Tensor | None = None) -> None:
+    """step = 0, pos = position and, given x, tok = token and x = embed[token], in one launch; see
+    solort_decode_start.  step/pos/tok int64 [1], embed [vocab, hidden] and x [hidden] bf16."""
+    for name, t in (("step", step), ("pos", pos)) + ((("tok", tok),) if x is not None else ()):
+        _need(t is not None and t.is_cuda and t.dtype == torch.int64 and t.is_contiguous() and t.numel() >= 1,
+              f"{name} must be int64 on the device")
+    vocab = stride = hidden = 0
+    if x is not None:
+        _on_gpu("embed", embed, torch.bfloat16)
+        _on_gpu("x", x, torch.bfloat16)
+        _need(embed.dim() == 2 and embed.stride(1) == 1, "embed must be [vocab, hidden] with unit column stride")
+        vocab, hidden = embed.shape
+        stride = embed.stride(0)
+        _need(x.numel() == hidden and x.is_contiguous(), f"x must hold hidden = {hidden} values")
+    rc = _lib.load().solort_decode_start(
+        int(token), int(position), None if x is None else embed.data_ptr(), vocab, stride, hidden,
+        None if x is None else x.data_ptr(), None if x is None else tok.data_ptr(), step.data_ptr(), pos.data_ptr(),
+        _stream(step))
+    _lib.check(rc, "decode_start")
+
+
 def greedy_advance(ws: torch.Tensor, vocab: int, embed: torch.Tensor, x: torch.Tensor, tok: torch.Tensor,
                    tokens: torch.Tensor | None, step: torch.Tensor, pos: torch.Tensor) -> None:
     """After gemv_argmax(..., out_idx=None, ws): tok = the argmax token, tokens[step] = tok (if step <

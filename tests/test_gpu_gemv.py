@@ -197,3 +197,20 @@ def test_greedy_advance_never_embeds_a_row_outside_the_table(gpu):
     assert step.item() == 2 and pos.item() == 31
     with pytest.raises(RuntimeError, match="outside the vocabulary"):
         ops.check_tokens(tokens.tolist(), n, "greedy decode")
+
+
+def test_decode_start(gpu):
+    """The chunk's first state equals the tensor ops it stands for; out-of-range tokens are refused."""
+    g = torch.Generator().manual_seed(3)
+    for vocab, hidden, pad in ((3, 8, 0), (100, 2560, 16), (7, 4104, 8)):
+        buf = torch.randn(vocab, hidden + pad, generator=g).to(torch.bfloat16).to(gpu)
+        embed = buf[:, :hidden]
+        tok, step, pos = (torch.full((1,), 9, dtype=torch.long, device=gpu) for _ in range(3))
+        x = torch.zeros(hidden, dtype=torch.bfloat16, device=gpu)
+        ops.decode_start(step, pos, 5)
+        assert (tok.item(), step.item(), pos.item()) == (9, 0, 5) and not x.any()
+        ops.decode_start(step, pos, 17, vocab - 1, embed, x, tok)
+        assert (tok.item(), step.item(), pos.item()) == (vocab - 1, 0, 17) and torch.equal(x, embed[vocab - 1])
+        for bad in (-1, vocab):
+            with pytest.raises(RuntimeError):
+                ops.decode_start(step, pos, 0, bad, embed, x, tok)
