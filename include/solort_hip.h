@@ -494,6 +494,15 @@ int solort_greedy_advance(const void* ws, int vocab, const void* embed, int64_t 
                           solort_stream_t stream);
 
 /*
+ * A step's inputs into its graph's static buffers, in one launch: bytes_i (a
+ * multiple of 4; 0: none) from src_i to dst_i, both 16-byte aligned and not
+ * overlapping, and *pos = position (cuda_graph_executor.py:195-206, :275-283).
+ */
+int solort_stage_inputs(void* dst0, const void* src0, int64_t bytes0, void* dst1, const void* src1, int64_t bytes1,
+                        void* dst2, const void* src2, int64_t bytes2, int64_t* pos, int64_t position,
+                        solort_stream_t stream);
+
+/*
  * The state a greedy chunk starts from, in one launch: *step = 0, *pos =
  * position, and with x non-NULL *tok = token and x [hidden] = embed row token
  * (cuda_graph_executor.py:165, :362-374).  Buffers as in solort_greedy_advance;

@@ -132,6 +132,10 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
         c_int, [c_void_p, c_int, c_void_p, c_int64, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
                 c_void_p],
     ),
+    "solort_stage_inputs": (
+        c_int, [c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_void_p,
+                c_int64, c_void_p]
+    ),
     "solort_decode_start": (
         c_int, [c_int64, c_int64, c_void_p, c_int, c_int64, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]
     ),

@@ -777,6 +777,25 @@ def gemv_argmax(w: torch.Tensor, x: torch.Tensor, out_idx: torch.Tensor | None, 
     _lib.check(rc, "gemv_argmax")
 
 
+def stage_inputs(pairs: list[tuple[torch.Tensor, torch.Tensor]], pos: torch.Tensor, position: int) -> None:
+    """dst.copy_(src) of up to three (dst, src) pairs and pos.fill_(position), in one launch where a source is a
+    contiguous tensor like its destination; others are copied by themselves.  See solort_stage_inputs."""
+    _need(len(pairs) <= 3, "at most three tensors")
+    _need(pos.is_cuda and pos.dtype == torch.int64 and pos.numel() == 1, "pos must be int64 [1] on the device")
+    args: list = []
+    for dst, src in pairs:
+        if (src.shape == dst.shape and src.dtype == dst.dtype and src.device == dst.device and src.is_contiguous()
+                and dst.is_contiguous() and src.data_ptr() % 16 == 0 and dst.data_ptr() % 16 == 0
+                and dst.numel() * dst.element_size() % 4 == 0 and not src.is_conj() and not src.is_neg()):
+            if src.data_ptr() != dst.data_ptr():
+                args += [dst.data_ptr(), src.data_ptr(), dst.numel() * dst.element_size()]
+        else:
+            dst.copy_(src)
+    args += [None, None, 0] * (3 - len(args) // 3)
+    rc = _lib.load().solort_stage_inputs(*args, pos.data_ptr(), int(position), _stream(pos))
+    _lib.check(rc, "stage_inputs")
+
+
 def decode_start(step: torch.Tensor, pos: torch.Tensor, position: int, token: int = 0,
                  embed: torch.Tensor | None = None, x: torch.Tensor | None = None,
                  tok: torch.Tensor | None = None) -> None:

@@ -192,15 +192,19 @@ class GraphQwen3Attention:
         """One decode step at `pos`: qkv [layers, 1, (nh+2nkv)*128] -> ctx [layers, 1, nh*128] (static buffer)."""
         if not 0 <= pos < self.max_len:
             raise RuntimeError(f"decode position {pos} outside [0, {self.max_len})")
-        self.qkv_dec.copy_(qkv)
-        self.pos_buf.fill_(int(pos))
+        return self._decode(qkv, pos, None)
+
+    def _decode(self, qkv: torch.Tensor, pos: int, logits: torch.Tensor | None) -> torch.Tensor:
+        pairs = [(self.qkv_dec, qkv)] + ([] if logits is None else [(self.logits_dec, logits)])
+        ops.stage_inputs(pairs, self.pos_buf, pos)
         self._replay(pos)
         return self.ctx_dec
 
     def decode_argmax(self, qkv: torch.Tensor, pos: int, logits: torch.Tensor) -> torch.Tensor:
         """decode() plus the in-graph greedy argmax of `logits` [1, vocab]; returns the [1] token buffer."""
-        self.logits_dec.copy_(logits)
-        self.decode(qkv, pos)
+        if not 0 <= pos < self.max_len:
+            raise RuntimeError(f"decode position {pos} outside [0, {self.max_len})")
+        self._decode(qkv, pos, logits)
         return self.tok_dec
 
     # ------------------------------------------------------------ prefill
@@ -280,11 +284,7 @@ class GraphQwen3Attention:
             with torch.cuda.graph(graph):
                 self._verify_forward(bound)
             self._ver_graphs[bound] = graph
-        self.qkv_ver.copy_(qkv)
-        if logits is not None:
-            self.logits_ver.copy_(logits)
-        if draft is not None:
-            self.draft_ver.copy_(draft)
-        self.vpos0.fill_(int(pos_start))
+        given = ((self.qkv_ver, qkv), (self.logits_ver, logits), (self.draft_ver, draft))
+        ops.stage_inputs([(dst, src) for dst, src in given if src is not None], self.vpos0, pos_start)
         self._ver_graphs[bound].replay()
         return self.ctx_ver
