@@ -149,7 +149,7 @@ class GraphQwen3Attention:
         # prefill: padded prompt rows per layer, bucketed graphs
         pmax = self.pre_buckets[-1]
         self.qkv_pre = torch.zeros(layers, pmax, self.width, dtype=torch.bfloat16, device=self.dev)
-        self.src_pre = ops.qkv_src(self.dev)  # where the fused layers' graph finds the prompt's qkv rows
+        self.src_pre: torch.Tensor | None = None  # where the fused layers' graphs find the prompt's qkv rows
         self.zero_pos = torch.zeros(1, dtype=torch.long, device=self.dev)  # prefill positions start at 0
         self.cs_pre = torch.zeros(2 * pmax * (HD // 2), dtype=torch.bfloat16, device=self.dev)  # step cos/sin
         self.ctx_pre = torch.zeros(layers, pmax, nh * HD, dtype=torch.bfloat16, device=self.dev)
@@ -239,20 +239,26 @@ class GraphQwen3Attention:
         bound = next((b for b in self.pre_buckets if b >= plen), None)
         if bound is None or plen < 1:
             raise RuntimeError(f"prompt length {plen} outside the prefill buckets {self.pre_buckets}")
-        if bound >= FUSED_PREFILL_MIN and self._rows_fit(qkv):
-            ops.set_qkv_src(self.src_pre, qkv)  # the replay reads the caller's rows
-            qkv.record_stream(torch.cuda.current_stream(qkv.device))
-        else:
+        # From FUSED_PREFILL_MIN rows on the replay reads the caller's rows where it can; the record points back to
+        # the runner's own buffer before this returns, so that nothing refers to the caller's memory afterwards.
+        fused = bound >= FUSED_PREFILL_MIN
+        direct = fused and self._rows_fit(qkv)
+        if not direct:
             self.qkv_pre[:, :plen].copy_(qkv)
             self.qkv_pre[:, plen:bound].zero_()
-            if bound >= FUSED_PREFILL_MIN:
-                ops.set_qkv_src(self.src_pre, self.qkv_pre[:, :plen])
+        if fused and self.src_pre is None:
+            self.src_pre = ops.qkv_src(self.kc.device)
         if bound not in self._pre_graphs:
             graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(graph):
                 self._prefill_forward(bound)
             self._pre_graphs[bound] = graph
+        if fused:
+            ops.set_qkv_src(self.src_pre, qkv if direct else self.qkv_pre[:, :plen])
         self._pre_graphs[bound].replay()
+        if direct:
+            qkv.record_stream(torch.cuda.current_stream(qkv.device))
+            ops.set_qkv_src(self.src_pre, self.qkv_pre)
         return self.ctx_pre[:, :plen]
 
     # ------------------------------------------------------------ verify

@@ -59,6 +59,7 @@ def test_runner_prefill_forms(gpu, plen, nh, nkv, form):
         assert torch.equal(got, want), again
         assert torch.equal(r.kc[:, :bound], kc) and torch.equal(r.vc[:, :bound], vc)
         assert (r.kc[:, bound:] == 5).all() and (r.vc[:, bound:] == 5).all()
+    assert r.src_pre[0].item() == r.qkv_pre.data_ptr()  # nothing refers to the caller's rows after the call
     other = torch.randn(L, plen - 1, width, generator=g).to(torch.bfloat16).to(gpu)  # other rows, the same graph
     assert torch.equal(r.prefill(other), _want(other, bound if plen - 1 > bound // 2 else bound // 2, nh, nkv, qn, kn)[0])
 
