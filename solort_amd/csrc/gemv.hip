@@ -14,7 +14,7 @@
 // output (_rmsnorm :25-28: fp32 x * rsqrt(mean(x^2) + eps), * fp32 w, to
 // bf16), the product, silu(gate), silu(gate) * up and the residual sum.
 //
-// Mapping: a workgroup (4 wavefronts) first stages x into LDS, normalised
+// Mapping: a workgroup (4 wavefronts, or 5: launch_gemv) first stages x into LDS, normalised
 // when NORM (every workgroup recomputes the 1-row norm: K <= 16384, a few KB
 // from L2), then each wavefront streams R weight rows: lane l takes the
 // 16-byte chunks l, l + 64, ... of each row (1 KB per row per instruction,
@@ -43,8 +43,8 @@ __device__ __forceinline__ float silu_bf16(float g) { return rbf(g / (1.0f + __e
 // The arguments the first loads need lead (w .. norm_w: 13 dwords), so they
 // arrive preloaded in SGPRs and the weight stream starts without waiting for
 // the kernel-argument fetch.
-template <int R, int U, int EPI, bool NORM>
-__global__ __launch_bounds__(256) void gemv_kernel(const uint16_t* __restrict__ w, int64_t w_stride, int n_out,
+template <int R, int U, int EPI, bool NORM, int NW = 4>
+__global__ __launch_bounds__(64 * NW) void gemv_kernel(const uint16_t* __restrict__ w, int64_t w_stride, int n_out,
                                                    int K, int64_t inter, const uint16_t* __restrict__ x,
                                                    const uint16_t* __restrict__ norm_w, float eps,
                                                    const uint16_t* res, uint16_t* out, uint64_t* arg_ws,
@@ -59,7 +59,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(const uint16_t* __restrict__ 
   // This wavefront's R weight rows; lane l streams their 16-byte chunks
   // l + 64 i, U chunks per row in flight.
   constexpr int NO = EPI == kGemvSwiglu ? R / 2 : R;  // outputs per wavefront
-  const int o0 = (blockIdx.x * 4 + wave) * NO;
+  const int o0 = (blockIdx.x * NW + wave) * NO;
   const uint16_t* rows[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
@@ -82,7 +82,13 @@ __global__ __launch_bounds__(256) void gemv_kernel(const uint16_t* __restrict__ 
   SOLORT_GEMV_LOADS(lane)
 
   // x into LDS (normalised: sum of squares in fp32, one block reduction).
-  gemv_stage_x<NORM>(x, norm_w, eps, K, sx, s_red);
+  if constexpr (NW == 4) {
+    gemv_stage_x<NORM>(x, norm_w, eps, K, sx, s_red);
+  } else {
+    static_assert(!NORM && EPI != kGemvArgmax, "the norm and the keys meet over four wavefronts");
+    for (int i = tid; i < nch; i += 64 * NW) sx[i] = *reinterpret_cast<const uint4*>(x + 8 * i);
+    __syncthreads();
+  }
 
   float acc[R];
 #pragma unroll
@@ -289,6 +295,24 @@ int launch_gemv(const char* name, const void* w, int64_t w_row_stride, int n_out
     else if (U == 8) SOLORT_GEMV_U(RR, 8, EE, NN);           \
     else SOLORT_GEMV_U(1, 20, EE, NN); /* U = 20 only with R = 1 */ \
   } while (0)
+  // A CU works on its workgroups at one rate, so the launch takes as long as the fullest CU: five wavefronts a
+  // workgroup where they make that one less full (N = 2560: two workgroups of five rows on every CU, 10 rows, instead
+  // of 12 on half of them: gate_up and down of 12 layers 341.7 -> 337.8 us; one token of 8 layers, o_proj too, 530.8
+  // -> 526.4).
+  const int cus = cu_count() > 0 ? cu_count() : 256;
+  const auto fullest = [&](int nw) { return ((n_out + nw - 1) / nw + cus - 1) / cus * nw; };
+  if (mode == kGemvResid && !norm && R == 1 && fullest(5) < fullest(4)) {
+    const dim3 grid((unsigned)((n_out + 4) / 5));
+#define SOLORT_GEMV_5(UU)                                                                                              \
+  hipLaunchKernelGGL((gemv_kernel<1, UU, kGemvResid, false, 5>), grid, dim3(320), lds, s, (const uint16_t*)w,         \
+                     w_row_stride, n_out, k, inter, (const uint16_t*)x, (const uint16_t*)nullptr, eps,                \
+                     (const uint16_t*)res, (uint16_t*)out, arg_ws, arg_idx)
+    if (U == 5) SOLORT_GEMV_5(5);
+    else if (U == 8) SOLORT_GEMV_5(8);
+    else SOLORT_GEMV_5(20);
+#undef SOLORT_GEMV_5
+    return check_launch(name);
+  }
 #define SOLORT_GEMV_R(EE, NN)        \
   switch (R) {                       \
     case 1: SOLORT_GEMV(1, EE, NN); break; \

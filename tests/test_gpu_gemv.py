@@ -214,3 +214,24 @@ def test_decode_start(gpu):
         for bad in (-1, vocab):
             with pytest.raises(RuntimeError):
                 ops.decode_start(step, pos, 0, bad, embed, x, tok)
+
+
+@pytest.mark.parametrize("n,k", [(2560, 4096), (2563, 9728), (1281, 72), (3328, 2560)])
+def test_gemv_residual_even_rows_per_cu(gpu, n, k):
+    """Row counts that five wavefronts a workgroup deal out more evenly than four, and one that they do not: the
+    bits of the same rows computed in slices of 64 (which stay with four)."""
+    print(f"[gemv even rows n={n} k={k}]", flush=True)
+    g = torch.Generator().manual_seed(n + k)
+    w = (torch.randn(n, k, generator=g) * 0.02).to(torch.bfloat16).to(gpu)
+    x, res = torch.randn(k, generator=g).to(torch.bfloat16).to(gpu), torch.randn(n, generator=g).to(torch.bfloat16).to(gpu)
+    got, want = torch.empty_like(res), torch.empty_like(res)
+    ops.gemv(w, x, got, res=res, mode=ops.GEMV_RESID)
+    for i in range(0, n, 64):
+        m = min(64, n - i)
+        part = torch.empty(m, dtype=torch.bfloat16, device=gpu)
+        ops.gemv(w[i:i + m], x, part, res=res[i:i + m].contiguous(), mode=ops.GEMV_RESID)
+        want[i:i + m] = part
+    assert torch.equal(got, want)
+    lin = (x.double().cpu() @ w.double().cpu().t()).to(torch.bfloat16).double()
+    exact = res.double().cpu() + lin
+    assert ((got.double().cpu() - exact).abs() <= exact.abs() * 2 ** -6 + 2e-3 + lin.abs() * 2 ** -7).all()
