@@ -7,7 +7,8 @@
 // (src/solort/model/cuda_graph_executor.py:115, :131-134), rounding where the
 // reference's bf16 tensors round.
 //
-// Bound: up to 256 rows the weight stream, from there the matrix units.  A
+// Bound: up to 256 rows what a CU can load, beyond loads and matrix units alike
+// (down of 1024 rows 60.9 us, loads alone 49.6, arithmetic alone 43.3).  A
 // workgroup takes a BM x BN tile over a share of k, WM x WN wavefronts of
 // v_mfma_f32_16x16x32_bf16 each BM / WM rows x BN / WN weight rows (A = W, B =
 // X, so a lane ends with four neighbouring outputs of one row).
@@ -16,11 +17,14 @@
 // barrier a stage.  Each stage buffer is an array of its own: the compiler then
 // sees that a stage's reads do not touch the buffers being filled and adds no
 // full wait.  A row's 16-byte chunks are stored in the order chunk ^ (row %
-// chunks) (rows of four chunks: row / 2), by permuting the lanes' source addresses, so the 16 rows of an
-// operand read fall on different banks.
-// A CU sustains about 35 GB/s of such loads whatever their depth, so the tile is
-// chosen to give every CU one workgroup and few repeated reads of X (launches of
-// 300 workgroups instead of 200: gate_up of 128 rows 44 us instead of 32); where
+// chunks) (rows of four chunks: row / 2), by permuting the lanes' source
+// addresses, so the 16 rows of an operand read fall on different banks.
+// Up to 256 rows the loads are the time (gate_up of 128 rows 32.3 us, its loads
+// alone 31.7, its arithmetic alone 19.8), and those of X and W add up (X alone
+// 10.3, W alone 21.6): a CU's requests return in order, so rows of X that hit
+// the L2 wait behind weights from HBM, and more stages in flight change
+// nothing.  The tile is therefore chosen to give every CU one workgroup and few
+// repeated reads of X (304 workgroups instead of 203: 44 us instead of 32); where
 // the tiles of N alone leave CUs idle (N = 2560: 40 tiles), k is split.
 // Workgroups that share a tile of W run on one XCD (block index mod 8).
 // Measured on MI355X, Qwen3-4B widths, graphs over 10 weight copies, 32 / 128 /
@@ -37,7 +41,6 @@ enum { kTilePlain = 0, kTileSwiglu = 1, kTileParts = 2 };
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
-
 
 typedef __attribute__((address_space(3))) void lds_void;
 
