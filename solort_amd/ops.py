@@ -27,6 +27,15 @@ def _stream(t: torch.Tensor) -> int:
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
+def _launch_on(t: torch.Tensor, name: str, *args) -> None:
+    """Calls solort_<name>(*args, stream) with t's device current, whichever device the caller has current: for the
+    launches that stand in for copies, fills and graph replays, which torch runs on their tensors' device (the
+    default stream's handle is 0 on every device, so the stream alone does not name one)."""
+    with torch.cuda.device(t.device):
+        rc = getattr(_lib.load(), "solort_" + name)(*args, _stream(t))
+        _lib.check(rc, name)
+
+
 def _need(cond: bool, msg: str) -> None:
     if not cond:
         raise RuntimeError(msg)
@@ -491,9 +500,8 @@ def set_qkv_src(src: torch.Tensor, qkv: torch.Tensor) -> None:
     _need(src.shape == (4,) and src.is_contiguous(), "src must be a qkv_src record")
     _on_gpu("qkv", qkv, torch.bfloat16)
     _need(qkv_src_takes(qkv, src.device), "qkv must be [layers, rows, width] bf16 rows, strides multiples of 8")
-    rc = _lib.load().solort_set_qkv_src(src.data_ptr(), qkv.data_ptr(), qkv.stride(0), qkv.stride(1), qkv.shape[1],
-                                        qkv.shape[2], _stream(src))
-    _lib.check(rc, "set_qkv_src")
+    _launch_on(src, "set_qkv_src", src.data_ptr(), qkv.data_ptr(), qkv.stride(0), qkv.stride(1), qkv.shape[1],
+               qkv.shape[2])
 
 
 def prefill_layer_src(src: torch.Tensor, layer: int, qn_w: torch.Tensor, kn_w: torch.Tensor, eps: float,
@@ -792,8 +800,7 @@ def stage_inputs(pairs: list[tuple[torch.Tensor, torch.Tensor]], pos: torch.Tens
         else:
             dst.copy_(src)
     args += [None, None, 0] * (3 - len(args) // 3)
-    rc = _lib.load().solort_stage_inputs(*args, pos.data_ptr(), int(position), _stream(pos))
-    _lib.check(rc, "stage_inputs")
+    _launch_on(pos, "stage_inputs", *args, pos.data_ptr(), int(position))
 
 
 def decode_start(step: torch.Tensor, pos: torch.Tensor, position: int, token: int = 0,
@@ -812,11 +819,9 @@ def decode_start(step: torch.Tensor, pos: torch.Tensor, position: int, token: in
         vocab, hidden = embed.shape
         stride = embed.stride(0)
         _need(x.numel() == hidden and x.is_contiguous(), f"x must hold hidden = {hidden} values")
-    rc = _lib.load().solort_decode_start(
-        int(token), int(position), None if x is None else embed.data_ptr(), vocab, stride, hidden,
-        None if x is None else x.data_ptr(), None if x is None else tok.data_ptr(), step.data_ptr(), pos.data_ptr(),
-        _stream(step))
-    _lib.check(rc, "decode_start")
+    _launch_on(step, "decode_start", int(token), int(position), None if x is None else embed.data_ptr(), vocab, stride,
+               hidden, None if x is None else x.data_ptr(), None if x is None else tok.data_ptr(), step.data_ptr(),
+               pos.data_ptr())
 
 
 def greedy_advance(ws: torch.Tensor, vocab: int, embed: torch.Tensor, x: torch.Tensor, tok: torch.Tensor,

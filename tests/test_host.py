@@ -1,6 +1,10 @@
 """Host-side logic of the runner that needs no GPU."""
-import pytest
+from types import SimpleNamespace
 
+import pytest
+import torch
+
+from solort_amd import _lib, ops
 from solort_amd.runner import (DECODE_BUCKETS, PREFILL_BUCKETS, decode_qkv_splits, decode_splits, verify_bound,
                                verify_splits)
 
@@ -55,3 +59,41 @@ def test_bucket_tables_follow_reference():
     # cuda_graph_executor.py:75-77 and :83-85
     assert DECODE_BUCKETS == (128, 256, 512, 1024, 2048, 4096)
     assert PREFILL_BUCKETS == (16, 32, 64, 128, 256, 512, 1024)
+
+
+def test_input_launches_run_on_their_tensors_device(monkeypatch):
+    """stage_inputs, set_qkv_src and decode_start launch with their tensors' device current and on its stream, while
+    the caller has another one current (they stand in for torch copies, fills and graph replays)."""
+    current, launches = [0], []
+
+    class Device:
+        def __init__(self, device):
+            self.index = torch.device(device).index
+
+        def __enter__(self):
+            self.before, current[0] = current[0], self.index
+
+        def __exit__(self, *exc):
+            current[0] = self.before
+
+    class Library:
+        def __getattr__(self, name):
+            return lambda *args: launches.append((name, current[0], args[-1])) or 0
+
+    monkeypatch.setattr(torch.cuda, "device", Device)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda d: SimpleNamespace(cuda_stream=100 + torch.device(d).index))
+    monkeypatch.setattr(_lib, "load", Library)
+
+    def on_one(dtype, *shape):
+        strides = torch.empty(shape, device="meta").stride()
+        return SimpleNamespace(device=torch.device("cuda:1"), is_cuda=True, dtype=dtype, shape=torch.Size(shape),
+                               data_ptr=lambda: 4096, numel=lambda: torch.Size(shape).numel(), dim=lambda: len(shape),
+                               stride=lambda i: strides[i], is_contiguous=lambda: True)
+
+    i64 = on_one(torch.int64, 1)
+    ops.stage_inputs([], i64, 3)
+    ops.set_qkv_src(on_one(torch.int64, 4), on_one(torch.bfloat16, 2, 300, 1024))
+    ops.decode_start(i64, i64, 3)
+    ops.decode_start(i64, i64, 3, 5, on_one(torch.bfloat16, 64, 32), on_one(torch.bfloat16, 32), i64)
+    assert launches == [("solort_" + n, 1, 101) for n in ("stage_inputs", "set_qkv_src", "decode_start", "decode_start")]
+    assert current == [0]
