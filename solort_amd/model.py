@@ -90,17 +90,23 @@ PARTS_MAX_LONG = 6
 class _RowBuffers:
     """Intermediate rows of a prompt bucket's layers, and which kernel takes each product: up to
     GEMM_ROWS_MAX rows solort_gemm_rows (few), else solort_gemm_tile where its shape and TILE_*_MAX allow
-    (tile_qkv, tile_gu; o_parts and d_parts: the k shares of the o_proj and down products), else the GEMM
-    library."""
+    (tile_qkv, tile_gu; o_parts and d_parts: the k shares of the o_proj and down products) and its offsets
+    reach every layer's weight, else the GEMM library."""
 
-    def __init__(self, s: ModelShape, rows: int, dev: torch.device) -> None:
+    def __init__(self, w: RandomQwen3, rows: int, dev: torch.device) -> None:
+        s = w.shape
+
+        def reaches(weights: list[torch.Tensor], n: int) -> bool:
+            return all(ops.gemm_tile_addresses(t, n) for t in weights)
+
         bf = dict(dtype=torch.bfloat16, device=dev)
         self.few = rows <= ops.GEMM_ROWS_MAX
         self.act = torch.empty(rows, s.inter, **bf)
-        self.tile_qkv = not self.few and rows <= TILE_QKV_MAX and ops.gemm_tile_parts(rows, s.qkv_width, s.hidden) > 0
+        self.tile_qkv = (not self.few and rows <= TILE_QKV_MAX and reaches(w.wqkv, s.qkv_width)
+                         and ops.gemm_tile_parts(rows, s.qkv_width, s.hidden) > 0)
         cus = torch.cuda.get_device_properties(dev).multi_processor_count
         one_round = 3 * cus // 4 <= -(-rows // 256) * -(-s.inter // 160) <= cus
-        self.tile_gu = (not self.few and (rows <= TILE_GU_MAX or one_round)
+        self.tile_gu = (not self.few and (rows <= TILE_GU_MAX or one_round) and reaches(w.wgu, 2 * s.inter)
                         and ops.gemm_tile_parts(rows, s.inter, s.hidden) > 0)
         if self.few or self.tile_qkv:
             self.qkv = torch.empty(rows, s.qkv_width, **bf)
@@ -108,13 +114,13 @@ class _RowBuffers:
             return
         self.h = torch.empty(rows, s.hidden, **bf)
 
-        def parts(k: int) -> torch.Tensor | None:
-            n = ops.gemm_tile_parts(rows, s.hidden, k) if s.hidden <= 8192 else 0
+        def parts(weights: list[torch.Tensor], k: int) -> torch.Tensor | None:
+            n = ops.gemm_tile_parts(rows, s.hidden, k) if s.hidden <= 8192 and reaches(weights, s.hidden) else 0
             if n == 0 or (rows > 256 and n > PARTS_MAX_LONG):
                 return None
             return torch.empty(n, rows, s.hidden, dtype=torch.float32, device=dev)
 
-        self.o_parts, self.d_parts = parts(s.nh * HD), parts(s.inter)
+        self.o_parts, self.d_parts = parts(w.wo, s.nh * HD), parts(w.wd, s.inter)
 
 
 class GraphQwen3Decode:
@@ -248,7 +254,7 @@ class GraphQwen3Decode:
         cs = self.cs_pre[: 2 * bound * (HD // 2)].view(2, bound, HD // 2)
         ops.rope_rows(self.inv_freq, self.zero_pos, bound, cs)                  # :111
         x = w.embed.index_select(0, self.pre_tok[:bound])                       # :112
-        b = _RowBuffers(s, bound, self.dev)
+        b = _RowBuffers(w, bound, self.dev)
         ctx = self.ctx_pre[:bound]
         if not b.few:
             ops.add_rmsnorm(x, None, w.in_ln[0], self.eps, None, b.h)            # :114

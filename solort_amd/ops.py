@@ -723,6 +723,12 @@ def gemm_tile_parts(m: int, n: int, k: int) -> int:
     return int(_lib.load().solort_gemm_tile_parts(int(m), int(n), int(k)))
 
 
+def gemm_tile_addresses(w: torch.Tensor, rows: int) -> bool:
+    """Whether gemm_tile's 32-bit byte offsets reach `rows` weight rows of w where they lie (solort_gemm_tile refuses
+    the rest: 2 GiB and more)."""
+    return w.stride(0) <= ((1 << 30) - 65536) // rows
+
+
 def gemm_tile(w: torch.Tensor, x: torch.Tensor, out: torch.Tensor, mode: int = TILE_PLAIN, inter: int = 0) -> None:
     """x [m, k] W^T for a prompt bucket's rows: bf16 out [m, n] (TILE_SWIGLU: silu(gate) * up of rows i and
     inter + i of w), or with TILE_PARTS out [n_parts, m, n] fp32, the sums over n_parts shares of k that

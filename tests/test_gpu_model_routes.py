@@ -1,0 +1,80 @@
+"""The products a prompt's rows (GraphQwen3Decode.prefill) and a verify's tokens take by bucket, width and weight
+layout: each combination against the fp32 evaluation of the same model (oracle/ref.py) on the CPU.
+
+Bar: the logits and the K/V rows within 0.03 of the fp32 model's (2-norm of the difference over the 2-norm).  Two
+layers of bf16 roundings leave 0.014 to 0.022 whatever the order of the sums; a neighbouring layer's norm weight, a
+stale row or a residual left out moves them by 0.1 and more.  Each case states the products it means to run, so that
+it fails when a rule sends it elsewhere."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from oracle import ref
+from solort_amd import model as mdl
+
+pytestmark = pytest.mark.gpu
+SMALL = mdl.ModelShape("small", hidden=512, inter=1024, nh=8, nkv=2, layers=2, vocab=4096, tie_embeddings=False)
+
+
+def _f32(w) -> dict:
+    return {k: (v.float().cpu() if torch.is_tensor(v) else [t.float().cpu() for t in v]) for k, v in vars(w).items()
+            if k != "shape"}
+
+
+def _near(got: torch.Tensor, want: torch.Tensor, what: str) -> None:
+    rel = ((got.float().cpu() - want).norm() / want.norm()).item()
+    print(f"  {what}: {rel:.4f} of the fp32 model", flush=True)
+    assert rel <= 0.03, what
+
+
+def _route(monkeypatch) -> list:
+    """The _RowBuffers that the calls after this make."""
+    made = []
+
+    class Recorded(mdl._RowBuffers):
+        def __init__(self, *args) -> None:
+            super().__init__(*args)
+            made.append(self)
+
+    monkeypatch.setattr(mdl, "_RowBuffers", Recorded)
+    return made
+
+
+def _prefill_near(w, plen: int, max_len: int, seed: int) -> mdl.GraphQwen3Decode:
+    s = w.shape
+    m = mdl.GraphQwen3Decode(w, max_len)
+    ids = torch.randint(0, s.vocab, (plen,), generator=torch.Generator().manual_seed(seed)).tolist()
+    m.prefill(ids)
+    kc, vc = (torch.zeros(s.layers, max_len, s.nkv, 128) for _ in range(2))
+    want = ref.prefill_model(_f32(w), ids, kc, vc, s.nh, s.nkv)
+    _near(m.logits.view(-1), want, "logits")
+    _near(m.kc[:, :plen], kc[:, :plen], "K rows")
+    _near(m.vc[:, :plen], vc[:, :plen], "V rows")
+    first = m.logits.clone()
+    m.prefill(ids)  # the captured graph again: the same bits
+    assert torch.equal(m.logits, first)
+    return m
+
+
+def _spread(weights: list[torch.Tensor], stride: int) -> list[torch.Tensor]:
+    """The same rows, stride elements apart (in one buffer, side by side)."""
+    n, k = weights[0].shape
+    buf = torch.empty(n * stride, dtype=torch.bfloat16, device=weights[0].device)
+    out = [buf.as_strided((n, k), (stride, 1), i * k) for i in range(len(weights))]
+    for o, t in zip(out, weights):
+        o.copy_(t)
+    return out
+
+
+@pytest.mark.parametrize("plen", [40, 300])
+def test_prefill_takes_weights_past_32_bit_offsets(gpu, monkeypatch, plen):
+    """Weights of 2 GiB and more are the library's (solort_gemm_tile has 32-bit offsets)."""
+    print(f"[prefill of {plen} rows, weights past 2 GiB]", flush=True)
+    w = mdl.RandomQwen3(SMALL, gpu, seed=101)
+    for name in ("wqkv", "wo", "wgu", "wd"):
+        t = getattr(w, name)
+        setattr(w, name, _spread(t, ((1 << 30) // t[0].shape[0] // 8 + 1) * 8))
+    made = _route(monkeypatch)
+    _prefill_near(w, plen, 512, plen)
+    assert all(not b.tile_qkv and not b.tile_gu and b.o_parts is None and b.d_parts is None for b in made) and made

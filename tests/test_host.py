@@ -97,3 +97,17 @@ def test_input_launches_run_on_their_tensors_device(monkeypatch):
     ops.decode_start(i64, i64, 3, 5, on_one(torch.bfloat16, 64, 32), on_one(torch.bfloat16, 32), i64)
     assert launches == [("solort_" + n, 1, 101) for n in ("stage_inputs", "set_qkv_src", "decode_start", "decode_start")]
     assert current == [0]
+
+
+def test_gemm_tile_offset_limit():
+    """2^30 elements less a row's tail, as solort_gemm_tile checks it."""
+    rows = 1024
+    limit = ((1 << 30) - 65536) // rows
+    def at(stride):
+        return torch.empty(0, dtype=torch.bfloat16).as_strided((0, 64), (stride, 1))
+    assert ops.gemm_tile_addresses(at(limit), rows) and not ops.gemm_tile_addresses(at(limit + 1), rows)
+    lib = _lib.load()
+    p = 4096  # never read: refused before any launch
+    stride = (limit // 8 + 1) * 8
+    rc = lib.solort_gemm_tile(p, stride, rows, 512, p, 512, 16, ops.TILE_PLAIN, 0, 1, p, rows, None)
+    assert rc != 0 and b"32-bit" in lib.solort_last_error()
