@@ -75,6 +75,13 @@ class RandomQwen3:
         self.lm_head = self.embed if s.tie_embeddings else rnd(s.vocab, H)
 
 
+def _rmsnorm_rows(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
+    """cuda_graph_executor.py:25-28 over the rows of a prompt, as the reference's torch ops on the
+    device: fp32 upcast, x * rsqrt(mean(x^2) + eps), times w in fp32, cast back."""
+    xf = x.float()
+    return ((xf * torch.rsqrt(xf.square().mean(-1, keepdim=True) + eps)) * w.float()).to(x.dtype)
+
+
 # Rows up to which solort_gemm_tile takes the qkv and gate/up products.  Qwen3-4B, us, with the library's product
 # behind: qkv at 256 rows 20.2 (31.4), 512 30.1 (28.0); gate/up with SwiGLU at 256 rows 42 (47.2 and the SwiGLU's 5),
 # at 512 75 (56.7 and 8), at 1024 102 (106.5 and 10) where its 256 x 160 tiles make one round over the CUs.  o_proj
@@ -88,10 +95,12 @@ PARTS_MAX_LONG = 6
 
 
 class _RowBuffers:
-    """Intermediate rows of a prompt bucket's layers, and which kernel takes each product: up to
-    GEMM_ROWS_MAX rows solort_gemm_rows (few), else solort_gemm_tile where its shape and TILE_*_MAX allow
-    (tile_qkv, tile_gu; o_parts and d_parts: the k shares of the o_proj and down products) and its offsets
-    reach every layer's weight, else the GEMM library."""
+    """Intermediate rows of the layers of a prompt bucket or a verify, and which kernel takes each product.
+    general: a weight that the kernels do not read as it lies (ops.weight_rows_fit, norm_weight_fits: a width
+    that is no multiple of 8, strided or unaligned rows, norm weights of another type), and every product and
+    norm runs as torch ops.  Otherwise up to GEMM_ROWS_MAX rows solort_gemm_rows (few), else solort_gemm_tile
+    where its shape and TILE_*_MAX allow (tile_qkv, tile_gu; o_parts and d_parts: the k shares of the o_proj
+    and down products) and its offsets reach every layer's weight, else the GEMM library."""
 
     def __init__(self, w: RandomQwen3, rows: int, dev: torch.device) -> None:
         s = w.shape
@@ -100,7 +109,11 @@ class _RowBuffers:
             return all(ops.gemm_tile_addresses(t, n) for t in weights)
 
         bf = dict(dtype=torch.bfloat16, device=dev)
-        self.few = rows <= ops.GEMM_ROWS_MAX
+        self.general = not (all(ops.weight_rows_fit(t) for t in [*w.wqkv, *w.wo, *w.wgu, *w.wd])
+                            and all(ops.norm_weight_fits(t) for t in [*w.in_ln, *w.post_ln]))
+        self.few = not self.general and rows <= ops.GEMM_ROWS_MAX
+        if self.general:
+            return
         self.act = torch.empty(rows, s.inter, **bf)
         self.tile_qkv = (not self.few and rows <= TILE_QKV_MAX and reaches(w.wqkv, s.qkv_width)
                          and ops.gemm_tile_parts(rows, s.qkv_width, s.hidden) > 0)
@@ -256,7 +269,7 @@ class GraphQwen3Decode:
         x = w.embed.index_select(0, self.pre_tok[:bound])                       # :112
         b = _RowBuffers(w, bound, self.dev)
         ctx = self.ctx_pre[:bound]
-        if not b.few:
+        if not b.few and not b.general:
             ops.add_rmsnorm(x, None, w.in_ln[0], self.eps, None, b.h)            # :114
         for li in range(s.layers):
             qkv = self._qkv_rows(li, x, b)                                       # :115
@@ -271,8 +284,10 @@ class GraphQwen3Decode:
         return x
 
     def _qkv_rows(self, li: int, x: torch.Tensor, b: "_RowBuffers") -> torch.Tensor:
-        """Layer li's qkv rows: of x through its norm (few rows), or of the normalised b.h."""
+        """Layer li's qkv rows: of x through its norm (few rows, general), or of the normalised b.h."""
         w = self.w
+        if b.general:
+            return F.linear(_rmsnorm_rows(x, w.in_ln[li], self.eps), w.wqkv[li])
         if b.few:
             ops.gemm_rows(w.wqkv[li], x, b.qkv, w.in_ln[li], self.eps)
             return b.qkv
@@ -283,9 +298,14 @@ class GraphQwen3Decode:
 
     def _mlp_rows(self, li: int, x: torch.Tensor, b: "_RowBuffers", ctx: torch.Tensor) -> None:
         """The rest of layer li for the rows of ctx (cuda_graph_executor.py:131-134): x gains the
-        layer's two residual terms, and b.h (not with few rows) becomes the next layer's normalised
-        input."""
+        layer's two residual terms, and b.h (not with few rows or general) becomes the next layer's
+        normalised input."""
         s, w = self.s, self.w
+        if b.general:
+            x.add_(F.linear(ctx, w.wo[li]))
+            gate, up = F.linear(_rmsnorm_rows(x, w.post_ln[li], self.eps), w.wgu[li]).split(s.inter, dim=-1)
+            x.add_(F.linear(F.silu(gate) * up, w.wd[li]))
+            return
         if b.few:
             ops.gemm_rows(w.wo[li], ctx, x, res=x, mode=ops.GEMV_RESID)
             ops.gemm_rows(w.wgu[li], x, b.act, w.post_ln[li], self.eps, mode=ops.GEMV_SWIGLU, inter=s.inter)
@@ -360,24 +380,24 @@ class GraphQwen3Decode:
         return self._read_tokens(n)
 
     def _verify_forward(self, bound: int) -> torch.Tensor:
-        """cuda_graph_executor.py:245-268 for the k1 tokens in vtok at vpos0..vpos0+k1-1: solort_gemm_rows
-        on the k1 rows around solort_decode_layer (nq = k1: prologue, KV write, causal attention over
-        the bucket), the logits [k1, V], their argmax (:475) and the accepted-prefix rule (:476-481)
-        into acc_ver = [a, tg[a]]."""
+        """cuda_graph_executor.py:245-268 for the k1 tokens in vtok at vpos0..vpos0+k1-1: the k1-row
+        products (_qkv_rows, _mlp_rows; k1 <= 8, so solort_gemm_rows unless general) around
+        solort_decode_layer (nq = k1: prologue, KV write, causal attention over the bucket), the logits
+        [k1, V], their argmax (:475) and the accepted-prefix rule (:476-481) into acc_ver = [a, tg[a]]."""
         s, w = self.s, self.w
         ops.rope_rows(self.inv_freq, self.vpos0, self.k1, self.cs_ver)          # :248
         x = w.embed.index_select(0, self.vtok)                                  # :249
-        bf = dict(dtype=torch.bfloat16, device=self.dev)
-        qkv, act = torch.empty(self.k1, s.qkv_width, **bf), torch.empty(self.k1, s.inter, **bf)
-        logits = torch.empty(self.k1, s.vocab, **bf)
+        b = _RowBuffers(w, self.k1, self.dev)
         for li in range(s.layers):
-            ops.gemm_rows(w.wqkv[li], x, qkv, w.in_ln[li], self.eps)             # :252-253
+            qkv = self._qkv_rows(li, x, b)                                      # :252-253
             ops.decode_layer(qkv, w.qn[li], w.kn[li], self.eps, self.cs_ver, self.vpos0, self.kc[li], self.vc[li],
                              bound, self.scale, self.ws_ver, verify_splits(bound, s.nkv), self.ctx_ver, s.nh, s.nkv)
-            ops.gemm_rows(w.wo[li], self.ctx_ver, x, res=x, mode=ops.GEMV_RESID)  # :264
-            ops.gemm_rows(w.wgu[li], x, act, w.post_ln[li], self.eps, mode=ops.GEMV_SWIGLU, inter=s.inter)  # :265-266
-            ops.gemm_rows(w.wd[li], act, x, res=x, mode=ops.GEMV_RESID)          # :267
-        ops.gemm_rows(w.lm_head, x, logits, w.final_norm, self.eps)              # :268
+            self._mlp_rows(li, x, b, self.ctx_ver)                              # :264-267
+        if b.few and ops.weight_rows_fit(w.lm_head) and ops.norm_weight_fits(w.final_norm):      # :268
+            logits = torch.empty(self.k1, s.vocab, dtype=torch.bfloat16, device=self.dev)
+            ops.gemm_rows(w.lm_head, x, logits, w.final_norm, self.eps)
+        else:
+            logits = F.linear(_rmsnorm_rows(x, w.final_norm, self.eps), w.lm_head)
         ops.argmax_rows(logits, self.tok_ver, self.ws_argv)
         if self.k1 > 1:
             ops.accept_prefix(self.tok_ver, self.vtok[1:], self.acc_ver)

@@ -686,6 +686,17 @@ def gemv(w: torch.Tensor, x: torch.Tensor, out: torch.Tensor, norm_w: torch.Tens
 GEMM_ROWS_MAX = 16
 
 
+def weight_rows_fit(w: torch.Tensor) -> bool:
+    """Whether gemv, gemm_rows and gemm_tile can read w [n, k] where it lies: bf16 rows of 16-byte chunks."""
+    return (w.dtype == torch.bfloat16 and w.dim() == 2 and w.stride(1) == 1 and w.stride(0) % 8 == 0
+            and w.stride(0) >= w.shape[1] and w.data_ptr() % 16 == 0 and w.shape[1] % 8 == 0 and w.shape[1] <= 65536)
+
+
+def norm_weight_fits(w: torch.Tensor) -> bool:
+    """Whether the kernels with a fused RMSNorm can read its weight w where it lies."""
+    return w.dtype == torch.bfloat16 and w.is_contiguous() and w.data_ptr() % 16 == 0
+
+
 def gemm_rows(w: torch.Tensor, x: torch.Tensor, out: torch.Tensor, norm_w: torch.Tensor | None = None,
               eps: float = 1e-6, res: torch.Tensor | None = None, mode: int = GEMV_PLAIN, inter: int = 0) -> None:
     """gemv for the rows of x [m, k], m <= GEMM_ROWS_MAX: out [m, n] = x W^T with the same fused neighbours

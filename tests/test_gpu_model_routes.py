@@ -57,6 +57,25 @@ def _prefill_near(w, plen: int, max_len: int, seed: int) -> mdl.GraphQwen3Decode
     return m
 
 
+def _verify_near(w, p0: int, seed: int) -> mdl.GraphQwen3Decode:
+    s = w.shape
+    m = mdl.GraphQwen3Decode(w, 256)
+    g = torch.Generator().manual_seed(seed)
+    for c in (m.kc, m.vc):
+        c[:, :p0].copy_(torch.randn(s.layers, p0, s.nkv, 128, generator=g))
+    kc, vc = m.kc.float().cpu(), m.vc.float().cpu()
+    toks = torch.randint(0, s.vocab, (m.k1,), generator=g).tolist()
+    m.vtok.copy_(torch.tensor(toks, device=m.dev))
+    got = m.verify(p0)
+    want = ref.verify_model(_f32(w), toks, p0, kc, vc, s.nh, s.nkv)
+    _near(got, want, "logits")
+    _near(m.kc[:, p0:p0 + m.k1], kc[:, p0:p0 + m.k1], "K rows")
+    _near(m.vc[:, p0:p0 + m.k1], vc[:, p0:p0 + m.k1], "V rows")
+    first = got.clone()
+    assert torch.equal(m.verify(p0), first)
+    return m
+
+
 def _spread(weights: list[torch.Tensor], stride: int) -> list[torch.Tensor]:
     """The same rows, stride elements apart (in one buffer, side by side)."""
     n, k = weights[0].shape
@@ -78,3 +97,37 @@ def test_prefill_takes_weights_past_32_bit_offsets(gpu, monkeypatch, plen):
     made = _route(monkeypatch)
     _prefill_near(w, plen, 512, plen)
     assert all(not b.tile_qkv and not b.tile_gu and b.o_parts is None and b.d_parts is None for b in made) and made
+
+
+def _weights(gpu, form: str, seed: int):
+    odd = dict(hidden=100) if form == "hidden 100" else dict(inter=100) if form == "inter 100" else {}
+    shape = mdl.ModelShape(**{**vars(SMALL), **odd})
+    w = mdl.RandomQwen3(shape, gpu, seed=seed)
+    if form == "columns":  # stored as their transposes
+        for name in ("wqkv", "wo", "wgu", "wd"):
+            setattr(w, name, [t.t().contiguous().t() for t in getattr(w, name)])
+    elif form == "unaligned rows":
+        w.wgu = _spread(w.wgu, 2 * shape.hidden + 4)
+    elif form == "fp32 norms":
+        w.in_ln, w.post_ln = w.in_ln.float(), w.post_ln.float()
+    elif form == "head":
+        w.lm_head, w.final_norm = w.lm_head.t().contiguous().t(), w.final_norm.float()
+    return w
+
+
+# prefill ends with gemv_argmax, which needs hidden a multiple of 8 and takes the head's rows as they lie
+@pytest.mark.parametrize("form", ["inter 100", "columns", "unaligned rows", "fp32 norms"])
+@pytest.mark.parametrize("plen", [9, 40, 300])
+def test_prefill_takes_weights_the_kernels_do_not_read(gpu, monkeypatch, form, plen):
+    print(f"[prefill of {plen} rows, {form}]", flush=True)
+    made = _route(monkeypatch)
+    _prefill_near(_weights(gpu, form, 102), plen, 512, plen)
+    assert made and all(b.general for b in made)
+
+
+@pytest.mark.parametrize("form", ["hidden 100", "inter 100", "columns", "unaligned rows", "fp32 norms", "head"])
+def test_verify_takes_weights_the_kernels_do_not_read(gpu, monkeypatch, form):
+    print(f"[verify, {form}]", flush=True)
+    made = _route(monkeypatch)
+    _verify_near(_weights(gpu, form, 103), 60, 104)
+    assert made and all(b.general == (form != "head") for b in made)
