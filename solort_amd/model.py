@@ -205,7 +205,15 @@ class GraphQwen3Decode:
 
     def start(self, token: int, pos: int) -> None:
         """The first input: token at position pos (rows 0..pos-1 of the cache hold the context)."""
-        ops.decode_start(self.step, self.pos, pos, token, self.w.embed, self.x.view(-1), self.tok)  # with :165
+        e = self.w.embed
+        if ops.weight_rows_fit(e):
+            ops.decode_start(self.step, self.pos, pos, token, e, self.x.view(-1), self.tok)  # with :165
+        else:  # another layout than the kernel's 16-byte chunks of a row
+            if not 0 <= int(token) < e.shape[0]:
+                raise RuntimeError(f"token {token} outside the vocabulary {e.shape[0]}")
+            self.tok.fill_(int(token))
+            ops.decode_start(self.step, self.pos, pos)
+            torch.index_select(e, 0, self.tok, out=self.x)
 
     def _step(self, bound: int) -> None:
         """One token: cuda_graph_executor.py:163-190 from the x the previous step (or start) left,

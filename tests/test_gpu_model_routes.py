@@ -131,3 +131,16 @@ def test_verify_takes_weights_the_kernels_do_not_read(gpu, monkeypatch, form):
     made = _route(monkeypatch)
     _verify_near(_weights(gpu, form, 103), 60, 104)
     assert made and all(b.general == (form != "head") for b in made)
+
+
+def test_start_takes_any_embedding_layout(gpu):
+    """The separate-ops tail gathers the embedding row with torch, so it and start() take any strides."""
+    w = mdl.RandomQwen3(SMALL, gpu, seed=105)
+    want = mdl.GraphQwen3Decode(w, 256, fused_tail=False).generate(7, 0, 6)
+    w.embed = w.embed.t().contiguous().t()
+    m = mdl.GraphQwen3Decode(w, 256, fused_tail=False)
+    m.start(9, 3)
+    assert torch.equal(m.x, w.embed[9:10]) and [m.tok.item(), m.pos.item(), m.step.item()] == [9, 3, 0]
+    assert m.generate(7, 0, 6) == want
+    with pytest.raises(RuntimeError, match="outside the vocabulary"):
+        m.start(SMALL.vocab, 3)
