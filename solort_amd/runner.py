@@ -40,6 +40,15 @@ PREFILL_BUCKETS = (16, 32, 64, 128, 256, 512, 1024)
 # rows 30.1 against 26.6.
 FUSED_PREFILL_MIN = 256
 
+# Padding rows of a bucket from which on a prompt in the runner's own buffer (copied there, or filled in
+# by the caller) goes through the record too, whose kernels skip the query tiles past the prompt; below,
+# its graph has the buffer's address in it, since the load of the record ahead of a layer's first loads
+# costs more than the few tiles.  fp32 rows, so with their copy, 12 Qwen3-4B layers, us, own buffer
+# against record: 208 rows 160.4 and 167.6, 192 160.0 and 157.7, 512 228.1 and 237.9, 464 227.5 and
+# 234.9, 448 227.3 and 225.3, 1024 371.3 and 381.1, 976 371.5 and 380.4, 960 370.5 and 370.6, 700 (with
+# a 1024-row bucket) 358 and 323.
+SRC_PADDING_MIN = 64
+
 
 def decode_splits(bound: int, nkv: int) -> int:
     """Key splits per KV head for a decode bucket.  Up to 256 keys: 16 keys per split; 512 keys: 32
@@ -155,7 +164,8 @@ class GraphQwen3Attention:
         self.ctx_pre = torch.zeros(layers, pmax, nh * HD, dtype=torch.bfloat16, device=self.dev)
         # q of the short buckets (the fused layer does not materialise it)
         self.q_pre = torch.zeros(min(pmax, FUSED_PREFILL_MIN), nh, HD, dtype=torch.bfloat16, device=self.dev)
-        self._pre_graphs: dict[int, torch.cuda.CUDAGraph] = {}
+        self._pre_own: dict[int, torch.cuda.CUDAGraph] = {}  # over the rows of qkv_pre
+        self._pre_src: dict[int, torch.cuda.CUDAGraph] = {}  # over the rows src_pre points to
 
     # ------------------------------------------------------------ decode
 
@@ -209,14 +219,23 @@ class GraphQwen3Attention:
 
     # ------------------------------------------------------------ prefill
 
-    def _prefill_forward(self, bound: int) -> None:
-        """cuda_graph_executor.py:109-130 (attention part): rows 0..bound-1 at positions 0..bound-1."""
+    @property
+    def _pre_graphs(self) -> dict[int, torch.cuda.CUDAGraph]:
+        """The captured prompt buckets, over qkv_pre where there is that form."""
+        return {**self._pre_src, **self._pre_own}
+
+    def _prefill_forward(self, bound: int, by_src: bool) -> None:
+        """cuda_graph_executor.py:109-130 (attention part): rows 0..bound-1 at positions 0..bound-1, found through
+        src_pre (by_src) or in qkv_pre."""
         cs = self.cs_pre[: 2 * bound * (HD // 2)].view(2, bound, HD // 2)
         ops.rope_rows(self.inv_freq, self.zero_pos, bound, cs)  # cos/sin once per step (:111)
         for li in range(self.L):
-            if bound >= FUSED_PREFILL_MIN:  # prologue of the K/V rows, then attention normalising q itself
+            if by_src:  # prologue of the K/V rows, then attention normalising q itself
                 ops.prefill_layer_src(self.src_pre, li, self.qn_w[li], self.kn_w[li], self.eps, cs, self.kc[li],
                                       self.vc[li], self.scale, self.ctx_pre[li, :bound], self.nh, self.nkv)
+            elif bound >= FUSED_PREFILL_MIN:
+                ops.prefill_layer(self.qkv_pre[li, :bound], self.qn_w[li], self.kn_w[li], self.eps, cs, self.kc[li],
+                                  self.vc[li], self.scale, self.ctx_pre[li, :bound], self.nh, self.nkv)
             else:  # short prompts: the whole prologue, then attention on the materialised q
                 ops.qknorm_rope_kvwrite_cs(self.qkv_pre[li, :bound], self.qn_w[li], self.kn_w[li], self.eps, cs,
                                            None, self.q_pre[:bound], self.kc[li], self.vc[li], self.nh, self.nkv)
@@ -241,21 +260,26 @@ class GraphQwen3Attention:
             raise RuntimeError(f"prompt length {plen} outside the prefill buckets {self.pre_buckets}")
         # From FUSED_PREFILL_MIN rows on the replay reads the caller's rows where it can; the record points back to
         # the runner's own buffer before this returns, so that nothing refers to the caller's memory afterwards.
+        # Rows that are in qkv_pre, or have to be copied there, need the record only to skip the bucket's padding.
         fused = bound >= FUSED_PREFILL_MIN
-        direct = fused and self._rows_fit(qkv)
+        padded = fused and bound - plen >= SRC_PADDING_MIN
+        direct = fused and self._rows_fit(qkv) and (padded or qkv.data_ptr() != self.qkv_pre.data_ptr())
         if not direct:
             self.qkv_pre[:, :plen].copy_(qkv)
             self.qkv_pre[:, plen:bound].zero_()
+        by_src = direct or padded
         if fused and self.src_pre is None:
             self.src_pre = ops.qkv_src(self.kc.device)
-        if bound not in self._pre_graphs:
+            ops.set_qkv_src(self.src_pre, self.qkv_pre)
+        graphs = self._pre_src if by_src else self._pre_own
+        if bound not in graphs:
             graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(graph):
-                self._prefill_forward(bound)
-            self._pre_graphs[bound] = graph
-        if fused:
+                self._prefill_forward(bound, by_src)
+            graphs[bound] = graph
+        if by_src:
             ops.set_qkv_src(self.src_pre, qkv if direct else self.qkv_pre[:, :plen])
-        self._pre_graphs[bound].replay()
+        graphs[bound].replay()
         if direct:
             qkv.record_stream(torch.cuda.current_stream(qkv.device))
             ops.set_qkv_src(self.src_pre, self.qkv_pre)

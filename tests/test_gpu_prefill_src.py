@@ -70,3 +70,32 @@ def test_set_qkv_src_rejects(gpu):
     for bad in (rows[:, :, 4:], rows[:, ::1, ::2], rows.float(), rows[0], rows[:, :0]):
         with pytest.raises(RuntimeError):
             ops.set_qkv_src(src, bad)
+
+
+# full buckets, the ends of the two rules (256: 64 padding rows, 65 and 63), padding of most of a bucket
+@pytest.mark.parametrize("plen", [129, 191, 192, 193, 256, 448, 449, 512, 700, 961, 1024])
+@pytest.mark.parametrize("form", ["fp32", "own", "rows"])
+def test_runner_prefill_over_own_buffer(gpu, plen, form):
+    """A prompt in the runner's buffer (copied there, or put there by the caller) that nearly fills its bucket
+    replays a graph over the buffer itself, every other one the graph over the record; the two alternate on one runner
+    without touching each other's rows."""
+    print(f"[prefill own buffer plen={plen} form={form}]", flush=True)
+    L, nh, nkv = 2, 16, 8
+    g = torch.Generator().manual_seed(plen)
+    qn, kn = ((torch.randn(L, HD, generator=g) * 0.1 + 1).to(torch.bfloat16).to(gpu) for _ in range(2))
+    r = runner.GraphQwen3Attention(nh, nkv, L, 1024, qn, kn, EPS, THETA, gpu, 5, 1000)
+    bound = next(b for b in r.pre_buckets if b >= plen)
+    for again in range(3):
+        rows = torch.randn(L, plen, r.width, generator=g).to(torch.bfloat16).to(gpu)
+        want, kc, vc = _want(rows, bound, nh, nkv, qn, kn)
+        if form == "own":
+            r.qkv_pre.fill_(3.0)  # rows past the prompt are not the caller's to clear
+            r.qkv_pre[:, :plen].copy_(rows)
+        got = r.prefill({"fp32": lambda: rows.float(), "own": lambda: r.qkv_pre[:, :plen], "rows": lambda: rows}[form]())
+        assert torch.equal(got, want), again
+        assert torch.equal(r.kc[:, :bound], kc) and torch.equal(r.vc[:, :bound], vc)
+        other = torch.randn(L, bound - 100, r.width, generator=g).to(torch.bfloat16).to(gpu)  # over the record
+        assert torch.equal(r.prefill(other), _want(other, bound, nh, nkv, qn, kn)[0])
+        assert r.src_pre[0].item() == r.qkv_pre.data_ptr()
+    assert sorted(r._pre_own) == ([bound] if form != "rows" and bound - plen < 64 else [])
+    assert sorted(r._pre_src) == [bound]
