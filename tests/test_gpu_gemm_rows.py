@@ -85,3 +85,65 @@ def test_gemm_rows_rejects_bad_arguments(gpu):
                       torch.zeros(ops.GEMM_ROWS_MAX + 1, 32, dtype=torch.bfloat16, device=gpu))
     with pytest.raises(RuntimeError):
         ops.gemm_rows(w, w[:2], torch.zeros(2, 33, dtype=torch.bfloat16, device=gpu))
+
+
+# Several tiles per workgroup (more than 16 outputs a CU) in each form that keeps x resident in several batches: the
+# next tile's first batches load during this one, the sums alternate between two LDS buffers; last, two to four tiles
+# of a one-batch form with 9-16 rows
+@pytest.mark.parametrize("m,n,k", [(16, 6144, 4096), (9, 12301, 4096), (5, 4200, 9728), (8, 9001, 9728), (5, 4200, 12288),
+                                   (3, 8403, 12288), (16, 6144, 2560), (13, 17001, 1024), (11, 9728, 9728)])
+@pytest.mark.parametrize("norm", [False, True], ids=["plain", "norm"])
+def test_gemm_rows_several_tiles_per_workgroup(gpu, m, n, k, norm):
+    test_gemm_rows_plain_and_residual(gpu, m, n, k, norm)
+
+
+# the gate/up products of 9-16 rows at the three served widths (x resident, two row groups), and one row group
+@pytest.mark.parametrize("m,inter,k", [(16, 9728, 2560), (12, 3072, 1024), (16, 12288, 4096), (8, 12288, 4096)])
+@pytest.mark.parametrize("norm", [False, True], ids=["plain", "norm"])
+def test_gemm_rows_swiglu_widths(gpu, m, inter, k, norm):
+    print(f"[gemm_rows swiglu m={m} inter={inter} k={k} norm={norm}]", flush=True)
+    g = torch.Generator().manual_seed(m + inter)
+    w = (torch.randn(2 * inter, k, generator=g) * 0.02).to(torch.bfloat16)
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16)
+    nw = (torch.randn(k, generator=g) * 0.1 + 1).to(torch.bfloat16)
+    h = ref.rmsnorm(x, nw, 1e-6) if norm else x
+    gate, up = _lin(h, w).double().split(inter, -1)
+    out = torch.empty(m, inter, dtype=torch.bfloat16, device=gpu)
+    ops.gemm_rows(w.to(gpu), x.to(gpu), out, nw.to(gpu) if norm else None, 1e-6, mode=ops.GEMV_SWIGLU, inter=inter)
+    _close(out, (gate * torch.sigmoid(gate)).to(torch.bfloat16).double() * up)
+
+
+@pytest.mark.parametrize("m,n,k", [(5, 70, 136), (16, 6144, 2560), (16, 2560, 4096), (5, 4200, 9728), (11, 2560, 9728)])
+@pytest.mark.parametrize("mode", [ops.GEMV_PLAIN, ops.GEMV_RESID, ops.GEMV_SWIGLU], ids=["plain", "resid", "swiglu"])
+def test_gemm_rows_nan_and_infinity_stay_in_their_row(gpu, m, n, k, mode):
+    """A NaN or an infinity in a row of x or of w reaches its own row of results only, and what lies behind the rows
+    (NaN here) none: the others keep their bits."""
+    print(f"[gemm_rows nan m={m} n={n} k={k} mode={mode}]", flush=True)
+    g = torch.Generator().manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16)
+    w = (torch.randn(2 * n if mode == ops.GEMV_SWIGLU else n, k, generator=g) * 0.02).to(torch.bfloat16)
+    nw = torch.ones(k, dtype=torch.bfloat16, device=gpu)
+    res = torch.randn(m, n, generator=g).to(torch.bfloat16).to(gpu)
+
+    def run(x, w):
+        xd, wd = _wide(x, gpu, 8), _wide(w, gpu, 16)
+        xd._base[:, k:] = float("nan")
+        wd._base[:, k:] = float("nan")
+        out = torch.empty(m, n, dtype=torch.bfloat16, device=gpu)
+        ops.gemm_rows(wd, xd, out, nw, 1e-6, res=res if mode == ops.GEMV_RESID else None, mode=mode, inter=n)
+        return out
+
+    clean = run(x, w)
+    assert torch.isfinite(clean).all()
+    bad_x, bad_w = {m // 2: "nan", m - 1: "inf"}, {1: "inf", n - 1: "nan"}
+    for row, v in bad_x.items():
+        x[row, (7 * row + 3) % k] = float(v)
+    for row, v in bad_w.items():
+        w[row, (11 * row + k - 1) % k] = float(v)
+    got = run(x, w)
+    rows = [r for r in range(m) if r not in bad_x]
+    cols = [c for c in range(n) if c not in bad_w]
+    assert torch.equal(got[rows][:, cols], clean[rows][:, cols])
+    # the norm spreads a bad x over its row
+    assert not torch.isfinite(got[m // 2]).any() and not torch.isfinite(got[m - 1]).any()
+    assert not torch.isfinite(got[:, n - 1]).any()

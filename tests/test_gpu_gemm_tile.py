@@ -91,3 +91,38 @@ def test_gemm_tile_rejects_bad_arguments(gpu):
         ops.gemm_tile(w, x, out[:, :38])
     with pytest.raises(RuntimeError):
         ops.gemm_tile(w, x, torch.zeros(3, 40, 40, device=gpu), mode=ops.TILE_PARTS)
+
+
+@pytest.mark.parametrize("m,n,k", [(17, 68, 640), (64, 100, 2560), (100, 196, 1024), (200, 6148, 512), (300, 132, 640),
+                                   (1000, 260, 512)])
+@pytest.mark.parametrize("mode", [ops.TILE_PLAIN, ops.TILE_PARTS, ops.TILE_SWIGLU], ids=["plain", "parts", "swiglu"])
+def test_gemm_tile_nan_and_infinity_stay_in_their_row(gpu, m, n, k, mode):
+    """A NaN or an infinity in a row of x or of w reaches its own row of results only, and what lies behind the rows
+    (NaN here) none: the others keep their bits."""
+    print(f"[gemm_tile nan m={m} n={n} k={k} mode={mode}]", flush=True)
+    x, w = _inputs(m, 2 * n if mode == ops.TILE_SWIGLU else n, k)
+    s = ops.gemm_tile_parts(m, n, k)
+
+    def run(x, w):
+        xd, wd = _wide(x, gpu, 8), _wide(w, gpu, 16)
+        xd._base[:, k:] = float("nan")
+        wd._base[:, k:] = float("nan")
+        if mode == ops.TILE_PARTS:
+            out = torch.empty(s, m, n, device=gpu)
+        else:
+            out = torch.empty(m, n, dtype=torch.bfloat16, device=gpu)
+        ops.gemm_tile(wd, xd, out, mode=mode, inter=n)
+        return out if out.dim() == 3 else out[None]
+
+    clean = run(x, w)
+    assert torch.isfinite(clean).all()
+    bad_x, bad_w = {m // 2: "nan", m - 1: "inf"}, {1: "inf", n - 1: "nan"}
+    for row, v in bad_x.items():
+        x[row, (7 * row + 3) % k] = float(v)
+    for row, v in bad_w.items():
+        w[row, (11 * row + k - 1) % k] = float(v)
+    got = run(x, w)
+    rows = [r for r in range(m) if r not in bad_x]
+    cols = [c for c in range(n) if c not in bad_w]
+    assert torch.equal(got[:, rows][:, :, cols], clean[:, rows][:, :, cols])
+    assert not torch.isfinite(got[:, m // 2]).all(0).any() and not torch.isfinite(got[:, :, n - 1]).all(0).any()

@@ -136,8 +136,8 @@ def test_decode_steps_match_reference_ops(gpu, shape):
 @pytest.mark.parametrize("plen,max_len,shape", [(37, 256, TINY_UNTIED), (300, 512, TINY_UNTIED), (300, 512, TINY_G8)],
                          ids=["bucket64", "bucket512-fused", "g8-bucket512-fused"])
 def test_prompt_prefill_then_decode_match_reference_ops(gpu, plen, max_len, shape):
-    """Prompt prefill (cuda_graph_executor.py:104-161: library GEMMs around solort_prefill_layer or
-    the prologue + solort_prefill_attn) and the decode steps after it, against the CPU evaluations of
+    """Prompt prefill (cuda_graph_executor.py:104-161: the buckets' products around solort_prefill_layer
+    or the prologue + solort_prefill_attn) and the decode steps after it, against the CPU evaluations of
     the same model in bf16 and fp32.  The first token's logits and the KV rows of the prompt are
     held to the bf16 reference's own distance from the fp32 model (as the decode steps are); the
     first token is the device argmax of its logits and becomes the decode input at position plen;

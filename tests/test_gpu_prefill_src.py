@@ -99,3 +99,24 @@ def test_runner_prefill_over_own_buffer(gpu, plen, form):
         assert r.src_pre[0].item() == r.qkv_pre.data_ptr()
     assert sorted(r._pre_own) == ([bound] if form != "rows" and bound - plen < 64 else [])
     assert sorted(r._pre_src) == [bound]
+
+
+@pytest.mark.parametrize("plen,bound,nh,nkv", [(130, 256, 8, 8), (250, 256, 16, 8), (300, 512, 32, 8), (512, 512, 8, 1)])
+def test_prefill_layer_src_fp32_output(gpu, plen, bound, nh, nkv):
+    """The fp32 output over a record: the bits of solort_prefill_layer's over the padded rows."""
+    print(f"[prefill_layer_src fp32 plen={plen} bound={bound} nh={nh} nkv={nkv}]", flush=True)
+    g = torch.Generator().manual_seed(plen)
+    width = (nh + 2 * nkv) * HD
+    rows = torch.randn(2, plen, width, generator=g).to(torch.bfloat16).to(gpu)
+    qn, kn = ((torch.randn(HD, generator=g) * 0.1 + 1).to(torch.bfloat16).to(gpu) for _ in range(2))
+    cs = ops.rope_rows(ops.inv_freq(HD, THETA, gpu), torch.zeros(1, dtype=torch.long, device=gpu), bound)
+    src = ops.qkv_src(gpu)
+    ops.set_qkv_src(src, rows)
+    pad = torch.zeros(bound, width, dtype=torch.bfloat16, device=gpu)
+    for layer in range(2):
+        kc, vc, kc2, vc2 = (torch.full((bound, nkv, HD), 7.0, dtype=torch.bfloat16, device=gpu) for _ in range(4))
+        out, out2 = (torch.empty(bound, nh * HD, device=gpu) for _ in range(2))
+        ops.prefill_layer_src(src, layer, qn, kn, EPS, cs, kc, vc, HD ** -0.5, out, nh, nkv)
+        pad[:plen] = rows[layer]
+        ops.prefill_layer(pad, qn, kn, EPS, cs, kc2, vc2, HD ** -0.5, out2, nh, nkv)
+        assert torch.equal(out[:plen], out2[:plen]) and torch.equal(kc, kc2) and torch.equal(vc, vc2)

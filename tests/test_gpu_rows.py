@@ -67,3 +67,27 @@ def test_rows_reject_bad_arguments(gpu):
         ops.add_rmsnorm(x, x.clone(), w, 1e-6, None, x.clone())
     with pytest.raises(RuntimeError):
         ops.swiglu_rows(x, torch.zeros(2, 16, dtype=torch.bfloat16, device=gpu))
+
+
+def test_nan_and_infinity_stay_in_their_row(gpu):
+    """A row that holds a NaN or an infinity leaves the other rows' bits alone, in each of the three launches."""
+    g = torch.Generator().manual_seed(5)
+    m, k = 7, 2568
+    x, y, gu, nw = _randn(g, m, k), _randn(g, m, k), _randn(g, m, 2 * k), _randn(g, k)
+    parts = torch.randn(3, m, k, generator=g)
+
+    def run():
+        outs = [torch.empty(m, k, dtype=torch.bfloat16, device=gpu) for _ in range(5)]
+        ops.add_rmsnorm(x.to(gpu), y.to(gpu), nw.to(gpu), 1e-6, outs[0], outs[1])
+        ops.add_parts_rmsnorm(x.to(gpu), parts.to(gpu), nw.to(gpu), 1e-6, outs[2], outs[3])
+        ops.swiglu_rows(gu.to(gpu), outs[4])
+        return outs
+
+    clean = run()
+    for t in (y, gu, parts[1]):
+        t[2, 11], t[5, k - 1] = float("nan"), float("inf")
+    got = run()
+    rows = [0, 1, 3, 4, 6]
+    for a, b in zip(got, clean):
+        assert torch.equal(a[rows], b[rows]) and torch.isfinite(b).all()
+        assert not torch.isfinite(a[2, 11]) and not torch.isfinite(a[5]).all()
