@@ -206,8 +206,9 @@ class GraphQwen3Decode:
     def start(self, token: int, pos: int) -> None:
         """The first input: token at position pos (rows 0..pos-1 of the cache hold the context)."""
         e = self.w.embed
-        if ops.weight_rows_fit(e):
-            ops.decode_start(self.step, self.pos, pos, token, e, self.x.view(-1), self.tok)  # with :165
+        row, col = e.stride()
+        if col == 1 and row % 8 == 0 and self.s.hidden % 8 == 0 and e.data_ptr() % 16 == 0:
+            ops.decode_start(self.step, self.pos, pos, token, e, self.x, self.tok)  # with :165
         else:  # another layout than the kernel's 16-byte chunks of a row
             if not 0 <= int(token) < e.shape[0]:
                 raise RuntimeError(f"token {token} outside the vocabulary {e.shape[0]}")

@@ -31,9 +31,11 @@ def _launch_on(t: torch.Tensor, name: str, *args) -> None:
     """Calls solort_<name>(*args, stream) with t's device current, whichever device the caller has current: for the
     launches that stand in for copies, fills and graph replays, which torch runs on their tensors' device (the
     default stream's handle is 0 on every device, so the stream alone does not name one)."""
-    with torch.cuda.device(t.device):
-        rc = getattr(_lib.load(), "solort_" + name)(*args, _stream(t))
-        _lib.check(rc, name)
+    if torch.cuda.current_device() != t.device.index:
+        with torch.cuda.device(t.device):
+            return _launch_on(t, name, *args)
+    rc = getattr(_lib.load(), "solort_" + name)(*args, _stream(t))
+    _lib.check(rc, name)
 
 
 def _need(cond: bool, msg: str) -> None:
@@ -824,10 +826,10 @@ def decode_start(step: torch.Tensor, pos: torch.Tensor, position: int, token: in
                  embed: torch.Tensor | None = None, x: torch.Tensor | None = None,
                  tok: torch.Tensor | None = None) -> None:
     """step = 0, pos = position and, given x, tok = token and x = embed[token], in one launch; see
-    solort_decode_start.  step/pos/tok int64 [1], embed [vocab, hidden] and x [hidden] bf16."""
-    for name, t in (("step", step), ("pos", pos)) + ((("tok", tok),) if x is not None else ()):
+    solort_decode_start.  step/pos/tok int64 [1], embed [vocab, hidden] and x (hidden values) bf16."""
+    for t in (step, pos) if x is None else (step, pos, tok):
         _need(t is not None and t.is_cuda and t.dtype == torch.int64 and t.is_contiguous() and t.numel() >= 1,
-              f"{name} must be int64 on the device")
+              "step, pos and tok must be int64 on the device")
     vocab = stride = hidden = 0
     if x is not None:
         _on_gpu("embed", embed, torch.bfloat16)

@@ -81,6 +81,7 @@ def test_input_launches_run_on_their_tensors_device(monkeypatch):
             return lambda *args: launches.append((name, current[0], args[-1])) or 0
 
     monkeypatch.setattr(torch.cuda, "device", Device)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: current[0])
     monkeypatch.setattr(torch.cuda, "current_stream", lambda d: SimpleNamespace(cuda_stream=100 + torch.device(d).index))
     monkeypatch.setattr(_lib, "load", Library)
 
