@@ -337,8 +337,9 @@ int solort_prefill_attn(const void* q, int T, int nh, int nkv, int hd, const voi
  * attention kernel normalises the q rows it stages.  Two launches on
  * `stream` (the K/V rows, then the attention).  It saves the q round trip
  * through HBM but puts the q normalisation ahead of each attention
- * workgroup's first MFMA: on MI355X it wins from about 400 rows on (Qwen3-4B
- * shape, 1024 rows: 27.0 against 30.1 us per layer) and loses below.
+ * workgroup's first MFMA: on MI355X it wins from 256 rows on (Qwen3-4B shape,
+ * us per layer: 128 rows 9.24 against 9.18, 256 11.25 against 11.37, 512 16.1
+ * against 17.5).
  * qkv [T, qkv_row_stride] bf16 (q, k, v heads of each row); rope_cs [2, T, 64]
  * bf16 from solort_rope_rows(inv_freq, 64, pos0 = 0, T).  Other arguments as
  * in solort_qknorm_rope_kvwrite_cs and solort_prefill_attn.
@@ -355,8 +356,8 @@ int solort_prefill_layer(const void* qkv, int64_t qkv_row_stride, int T, int nh,
  * row t starts at qkv + l * layer_stride + t * row_stride (elements, multiples of
  * 8), t < rows, width elements each.  T is the graph's row count (its cos/sin
  * table has T rows): K/V rows 0..T-1 are written, those past the record's rows
- * as those of zero input, and out rows 0..rows-1.  The rows must stay valid until
- * the replay has run.
+ * as those of zero input, and out rows 0..rows-1.  The rows must stay valid and
+ * unmodified until the replay has run.
  */
 int solort_set_qkv_src(void* src, const void* qkv, int64_t layer_stride, int64_t row_stride, int64_t rows, int width,
                        solort_stream_t stream);

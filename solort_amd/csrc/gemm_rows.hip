@@ -27,8 +27,8 @@
 // RMSNorm: a lane holds the x it will multiply, so the sum of squares is
 // collected from those registers (one LDS exchange between the wavefronts)
 // while the weight loads are in flight.
-// One workgroup per CU: 256 registers a wavefront hold x and two batches of
-// weights, 80-160 KB in flight per CU.  (Two workgroups of 128 registers each
+// One workgroup per CU: 256 registers a wavefront hold x and two batches of U
+// steps of weights, 32 KB x U in flight per CU (K = 2560: U = 5, 160 KB).  (Two workgroups of 128 registers each
 // spill: gate_up 25-28 us instead of 18.5.)
 // Measured on MI355X, 5 rows, Qwen3-4B, graphs over 12 weight copies, with the
 // library product of the same shape (no fused neighbours) behind: qkv 7.9 us

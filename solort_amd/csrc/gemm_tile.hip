@@ -8,8 +8,8 @@
 // reference's bf16 tensors round.
 //
 // Bound: up to 256 rows what a CU can load, beyond loads and matrix units alike
-// (down of 1024 rows 60.9 us, loads alone 49.6, arithmetic alone 43.3).  A
-// workgroup takes a BM x BN tile over a share of k, WM x WN wavefronts of
+// (down of 1024 rows: its loads alone take 81 % of its time, its arithmetic
+// alone 71 %).  A workgroup takes a BM x BN tile over a share of k, WM x WN wavefronts of
 // v_mfma_f32_16x16x32_bf16 each BM / WM rows x BN / WN weight rows (A = W, B =
 // X, so a lane ends with four neighbouring outputs of one row).
 // Stages of kBK columns of X and W go from memory straight into LDS (16 bytes
@@ -27,11 +27,13 @@
 // repeated reads of X (304 workgroups instead of 203: 44 us instead of 32); where
 // the tiles of N alone leave CUs idle (N = 2560: 40 tiles), k is split.
 // Workgroups that share a tile of W run on one XCD (block index mod 8).
-// Measured on MI355X, Qwen3-4B widths, graphs over 10 weight copies, 32 / 128 /
-// 1024 rows, the library's product behind (us): qkv 10.0 / 16.6 / - (11.7 / 19.1
-// / 38.1), o_proj 5.8 / 7.8 / 25.4 (9.3 / 19.3 / 30.8), gate_up with SwiGLU 21.7
-// / 32.1 / 102 (24.6 / 31.2 / 106.5 without), down 11.8 / 17.7 / 51.5 (21.4 / 52.6
-// / 79.3).
+// Measured on MI355X, Qwen3-4B widths, normal random values, graphs over 10
+// weight copies with one x and one result, 32 / 128 / 1024 rows, the library's
+// product behind (us, two runs within 5 %): qkv 10.2 / 17.1 / - (12.0 / 19.2 /
+// 40.1), o_proj 5.9 / 8.2 / 28.3 (9.4 / 19.1 / 31.1), gate_up with SwiGLU 23.2 /
+// 32.3 / 96 (24.9 / 33.1 / 107 without), down 12.6 / 19.6 / 55 (21.4 / 52.6 /
+// 79).  The time depends on the values through the clock: down of 1024 rows
+// takes 49 us with zero weights.
 #include "common.h"
 #include "capi_internal.h"
 

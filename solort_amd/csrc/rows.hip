@@ -21,6 +21,7 @@
 
 namespace solort {
 
+// Rounded to bf16 the same as with expf, for each of the 65281 bf16 gates that are no NaN (compared one by one).
 __device__ __forceinline__ float silu_bf16_rows(float g) { return rbf(g / (1.0f + __expf(-g))); }
 
 // One 256-thread workgroup per row; a thread keeps its first kNormReg 16-byte
@@ -106,7 +107,7 @@ __global__ __launch_bounds__(256) void add_rmsnorm_kernel(const uint16_t* x, int
 
 // x_out = x + bf16(sum of the n_parts fp32 shares of y), h = _rmsnorm(x_out, w) (NORM): the end of a product whose
 // k was split over workgroups (solort_gemm_tile).  One workgroup per row, a thread per 16-byte chunk of the row (two
-// from k = 4096 on), so that a row's shares are all in flight at once; the shares are added in order.
+// above k = 4096), so that a row's shares are all in flight at once; the shares are added in order.
 template <bool NORM>
 __global__ __launch_bounds__(512) void add_parts_rmsnorm_kernel(const uint16_t* x, int64_t x_stride,
                                                                 const float* __restrict__ parts, int n_parts,

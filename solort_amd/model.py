@@ -83,10 +83,10 @@ def _rmsnorm_rows(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
 
 
 # Rows up to which solort_gemm_tile takes the qkv and gate/up products.  Qwen3-4B, us, with the library's product
-# behind: qkv at 256 rows 20.2 (31.4), 512 30.1 (28.0); gate/up with SwiGLU at 256 rows 42 (47.2 and the SwiGLU's 5),
-# at 512 75 (56.7 and 8), at 1024 102 (106.5 and 10) where its 256 x 160 tiles make one round over the CUs.  o_proj
-# and down, whose 2560 outputs alone do not fill the chip, take it at every size (1024 rows: 25.4 and 51.5, library
-# 30.8 and 79.3), unless over many rows the fp32 shares themselves are the cost: a Qwen3-0.6B layer, 8 shares of 1024
+# behind: qkv at 256 rows 20.7 (31.2), 512 37 (27.3); gate/up with SwiGLU at 256 rows 43 (47.2 and the SwiGLU's 5),
+# at 512 88 (59.5 and 8), at 1024 96 (107 and 10) where its 256 x 160 tiles make one round over the CUs.  o_proj
+# and down, whose 2560 outputs alone do not fill the chip, take it at every size (1024 rows: 28.3 and 55, library
+# 31.1 and 79), unless over many rows the fp32 shares themselves are the cost: a Qwen3-0.6B layer, 8 shares of 1024
 # outputs, 85.2 us at 512 rows and 111.7 at 1024, with the library 80.4 and 101.6 (Qwen3-4B, 6 shares at 512 rows:
 # 175.9, with the library 191.9).
 TILE_QKV_MAX = 256

@@ -8,11 +8,12 @@ lazily and routed by position (:75-77, :192-214), bucketed prefill graphs
 (:83-85, :137-161), a fixed K+1-token verify graph (:270-289) and the in-graph
 greedy argmax (:206).  Everything outside attention (embedding, QKV/o_proj
 GEMMs, MLP, lm_head) is not part of this library: each layer's fused QKV
-projection output is a static input buffer the caller fills (the role the
-QKV GEMM plays at :115, :171, :253), and each layer's attention output
-``ctx`` [T, nh*128] is left in a static output buffer (what o_proj consumes
-at :131, :185, :264).  Logits for the argmax are likewise a caller-filled
-buffer.
+projection output is an input the caller fills (the role the QKV GEMM plays at
+:115, :171, :253): copied into a static buffer, except that a prompt in a bucket
+from FUSED_PREFILL_MIN rows on is read from the caller's tensor by the replay;
+each layer's attention output ``ctx`` [T, nh*128] is left in a static output
+buffer (what o_proj consumes at :131, :185, :264).  Logits for the argmax are
+likewise given by the caller.
 
 Decode and verify run one launch per layer (solort_decode_layer: prologue,
 KV write, split-KV attention and combine); prefill runs the prologue launch
@@ -35,9 +36,10 @@ PREFILL_BUCKETS = (16, 32, 64, 128, 256, 512, 1024)
 # Prefill buckets from this length on use solort_prefill_layer (q normalised inside the attention
 # kernel); shorter ones the two-launch prologue + attention.  The fused layer saves the q round
 # trip through HBM and adds the normalisation work ahead of each attention workgroup's first MFMA.
-# Measured on MI355X, Qwen3-4B shape, graphed 36-layer step per layer (two-launch against fused):
-# 128 rows 9.28 against 9.40 us, 256 rows 11.64 against 11.43, 512 rows 17.83 against 16.28, 1024
-# rows 30.1 against 26.6.
+# Measured on MI355X, Qwen3-4B shape, graphed 36-layer step per layer, rows in qkv_pre (two-launch
+# against fused): 128 rows 9.18 against 9.24 us, 256 rows 11.37 against 11.25, 512 rows 17.52 against
+# 16.11.  Read through the record instead, so without the copy of the prompt, the fused layer takes
+# 12.4 us at 256 rows, 16.7 at 512 (512 rows of 12 layers with their copy: 217.8 -> 205.5 us).
 FUSED_PREFILL_MIN = 256
 
 # Padding rows of a bucket from which on a prompt in the runner's own buffer (copied there, or filled in
@@ -250,10 +252,11 @@ class GraphQwen3Attention:
 
     def prefill(self, qkv: torch.Tensor) -> torch.Tensor:
         """Graphed bucketed prefill (cuda_graph_executor.py:149-161): qkv [layers, plen, width] for
-        prompt positions 0..plen-1, padded with zero rows to the first bucket >= plen (from
-        FUSED_PREFILL_MIN on without a copy: the replay reads the rows of qkv itself).  Writes cache
-        rows 0..bucket-1 (padding rows included, as in the reference; decode never reads them) and
-        returns ctx [layers, plen, nh*128] (a view of the static buffer)."""
+        prompt positions 0..plen-1, padded with zero rows to the first bucket >= plen.  From
+        FUSED_PREFILL_MIN on bf16 rows are not copied: the replay, which may run after this returns,
+        reads qkv itself, so whatever rewrites qkv has to be ordered after the current stream.
+        Writes cache rows 0..bucket-1 (padding rows included, as in the reference; decode never
+        reads them) and returns ctx [layers, plen, nh*128] (a view of the static buffer)."""
         plen = int(qkv.shape[1])
         bound = next((b for b in self.pre_buckets if b >= plen), None)
         if bound is None or plen < 1:

@@ -91,3 +91,14 @@ def test_nan_and_infinity_stay_in_their_row(gpu):
     for a, b in zip(got, clean):
         assert torch.equal(a[rows], b[rows]) and torch.isfinite(b).all()
         assert not torch.isfinite(a[2, 11]) and not torch.isfinite(a[5]).all()
+
+
+def test_swiglu_rows_silu_of_every_gate(gpu):
+    """silu of each bf16 value, infinities included, rounds to the bits of torch's (up = 1)."""
+    gate = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(torch.bfloat16).to(gpu)
+    out = torch.empty(1, 65536, dtype=torch.bfloat16, device=gpu)
+    ops.swiglu_rows(torch.cat([gate, torch.ones_like(gate)])[None], out)
+    want = torch.nn.functional.silu(gate)[None]
+    assert torch.equal(out.isnan(), want.isnan())
+    ok = ~want.isnan()
+    assert torch.equal(out[ok].view(torch.int16), want[ok].view(torch.int16))
