@@ -109,8 +109,9 @@ class _RowBuffers:
             return all(ops.gemm_tile_addresses(t, n) for t in weights)
 
         bf = dict(dtype=torch.bfloat16, device=dev)
+        norms = [t for n in (w.in_ln, w.post_ln) for t in ([n] if torch.is_tensor(n) and n.is_contiguous() else n)]
         self.general = not (all(ops.weight_rows_fit(t) for t in [*w.wqkv, *w.wo, *w.wgu, *w.wd])
-                            and all(ops.norm_weight_fits(t) for t in [*w.in_ln, *w.post_ln]))
+                            and all(ops.norm_weight_fits(t) for t in norms))
         self.few = not self.general and rows <= ops.GEMM_ROWS_MAX
         if self.general:
             return

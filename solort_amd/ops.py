@@ -690,8 +690,10 @@ GEMM_ROWS_MAX = 16
 
 def weight_rows_fit(w: torch.Tensor) -> bool:
     """Whether gemv, gemm_rows and gemm_tile can read w [n, k] where it lies: bf16 rows of 16-byte chunks."""
-    return (w.dtype == torch.bfloat16 and w.dim() == 2 and w.stride(1) == 1 and w.stride(0) % 8 == 0
-            and w.stride(0) >= w.shape[1] and w.data_ptr() % 16 == 0 and w.shape[1] % 8 == 0 and w.shape[1] <= 65536)
+    if w.dtype != torch.bfloat16 or w.dim() != 2:
+        return False
+    (row, col), k = w.stride(), w.shape[1]
+    return col == 1 and row % 8 == 0 and row >= k and k % 8 == 0 and k <= 65536 and w.data_ptr() % 16 == 0
 
 
 def norm_weight_fits(w: torch.Tensor) -> bool:
