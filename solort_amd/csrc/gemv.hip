@@ -298,10 +298,14 @@ int launch_gemv(const char* name, const void* w, int64_t w_row_stride, int n_out
   // A CU works on its workgroups at one rate, so the launch takes as long as the fullest CU: five wavefronts a
   // workgroup where they make that one less full (N = 2560: two workgroups of five rows on every CU, 10 rows, instead
   // of 12 on half of them: gate_up and down of 12 layers 341.7 -> 337.8 us; one token of 8 layers, o_proj too, 530.8
-  // -> 526.4).
+  // -> 526.4).  Not where fewer than an eighth of the CUs have that one workgroup more, nor for short rows, whose time
+  // is the launch: four and five wavefronts, us, N x K = 3073 x 9728 13.4 and 14.1, 2049 x 4096 5.43 and 5.54, 2304 x
+  // 1024 3.48 and 3.55; past the line 1152 x 4096 4.70 and 4.38, 2304 x 2560 4.80 and 4.54, 3500 x 9728 15.2 and 14.5
+  // (and one loss, 2560 x 12288: 13.9 and 14.2; 1152 to 3200 rows of 12288 gain 2 to 4 %).
   const int cus = cu_count() > 0 ? cu_count() : 256;
   const auto fullest = [&](int nw) { return ((n_out + nw - 1) / nw + cus - 1) / cus * nw; };
-  if (mode == kGemvResid && !norm && R == 1 && fullest(5) < fullest(4)) {
+  if (mode == kGemvResid && !norm && R == 1 && k >= 2048 && fullest(5) < fullest(4) &&
+      (n_out + 3) / 4 % cus * 8 >= cus) {
     const dim3 grid((unsigned)((n_out + 4) / 5));
 #define SOLORT_GEMV_5(UU)                                                                                              \
   hipLaunchKernelGGL((gemv_kernel<1, UU, kGemvResid, false, 5>), grid, dim3(320), lds, s, (const uint16_t*)w,         \

@@ -216,10 +216,12 @@ def test_decode_start(gpu):
                 ops.decode_start(step, pos, 0, bad, embed, x, tok)
 
 
-@pytest.mark.parametrize("n,k", [(2560, 4096), (2563, 9728), (1281, 72), (3328, 2560)])
+@pytest.mark.parametrize("n,k", [(2560, 4096), (2563, 9728), (1281, 72), (3328, 2560), (1152, 2048), (1148, 2048),
+                                 (2304, 2040), (3073, 2560)])
 def test_gemv_residual_even_rows_per_cu(gpu, n, k):
-    """Row counts that five wavefronts a workgroup deal out more evenly than four, and one that they do not: the
-    bits of the same rows computed in slices of 64 (which stay with four)."""
+    """Row counts that five wavefronts a workgroup deal out more evenly than four, and sizes on either side of the
+    rule's lines (rows, and an eighth of the CUs fuller): the bits of the same rows computed in slices of 64 (which
+    stay with four)."""
     print(f"[gemv even rows n={n} k={k}]", flush=True)
     g = torch.Generator().manual_seed(n + k)
     w = (torch.randn(n, k, generator=g) * 0.02).to(torch.bfloat16).to(gpu)
